@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from wisp import quant
+from wisp import kernels, quant
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -25,3 +25,24 @@ def test_quantize_group_128_edges(bits, n, dtype, shift):
     buf[shift:] = torch.from_numpy(w).to(DEV)
     got = quant.quantize(buf[shift:].view(3, n), bits, 128).cpu().numpy()
     assert np.array_equal(got, O.quantize(w, bits, 128))
+
+
+# capacities past 128 chunks of 64 positions merge with eight waves per head: the first 64 chunks by the lower four,
+# the rest by all of them, in batches of 16 per wave
+@pytest.mark.parametrize("Hq,Hk,D", [(8, 2, 128), (4, 2, 64), (2, 2, 256)])
+def test_attn_decode_wide_merge(Hq, Hk, D):
+    T = 128 * 64 + 64 * 70  # 198 chunks: 64, then 8 x 16, then 6
+    gen = torch.Generator(device=DEV).manual_seed(Hq + D)
+    q, k, v = (torch.randn(s, generator=gen, device=DEV).to(torch.bfloat16)
+               for s in ((1, Hq, 1, D), (1, Hk, T, D), (1, Hk, T, D)))
+    for pos in (0, 63, 64, 4095, 4096, 4159, 8191, 12287, 12288, T - 1):
+        p = torch.tensor([pos], device=DEV)
+        kn, vn = k.clone(), v.clone()
+        kn[:, :, pos + 1 :], vn[:, :, pos + 1 :] = float("nan"), float("nan")  # nothing past the position is read
+        got = kernels.attn_decode(q, kn, vn, p, D**-0.5).view(Hq, D).double()
+        kk = k[0, :, : pos + 1].double().repeat_interleave(Hq // Hk, 0)
+        vv = v[0, :, : pos + 1].double().repeat_interleave(Hq // Hk, 0)
+        w = ((kk @ q[0, :, 0].double()[:, :, None])[..., 0] * D**-0.5).softmax(-1)
+        ref = (w[:, None] @ vv)[:, 0]
+        # one bf16 rounding (2^-9 of a value at most) and fp32 sums
+        assert ((got - ref).norm() / ref.norm()).item() <= 2.0**-8, pos

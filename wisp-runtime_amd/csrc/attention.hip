@@ -25,6 +25,7 @@
 
 namespace wisp {
 
+constexpr int kMergeWide = 128;  // capacities of more chunks merge with 8 waves per head (below)
 constexpr int kChunk = 64;  // positions per k_attn_mfma workgroup (4 waves of 16)
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -295,18 +296,19 @@ __device__ __forceinline__ float row0_max(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
 }
 
-// One workgroup (4 waves) per query head: wave w merges chunks w, w+4, ... in
-// batches of 16 with a running maximum. Lane b < 16 reads the m and l of the batch's
+// One workgroup (NW = 4 or 8 waves) per query head: wave w < 4 merges chunks w, w+4, ...
+// of the first 64 in a batch of 16, and wave w < NW chunks 64 + w, 64 + w + NW, ... in
+// batches of 16, with a running maximum. Lane b < 16 reads the m and l of the batch's
 // chunk b and computes its weight (one exponential per chunk); the weights reach the
-// o sums of every lane through readlane. The four waves' sums are rescaled to the
+// o sums of every lane through readlane. The waves' sums are rescaled to the
 // common maximum in LDS. Only the chunks up to pos have records (pos read from device
 // memory, so graphs follow it).
-template <int D>
-__global__ __launch_bounds__(256) void k_attn_merge(const float* __restrict__ part, const int64_t* __restrict__ pos_ptr,
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW) void k_attn_merge(const float* __restrict__ part, const int64_t* __restrict__ pos_ptr,
                                                     int G, int nsplit, uint16_t* __restrict__ out) {
     constexpr int DPL = D / 64, B = 16;
-    __shared__ float red_m[4], red_l[4];
-    __shared__ float red_o[4][D];
+    __shared__ float red_m[NW], red_l[NW];
+    __shared__ float red_o[NW][D];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // chunk indices in SGPRs
     const int h = blockIdx.x, hk = h / G, g = h - hk * G;
     const int64_t pos = *pos_ptr;
@@ -319,16 +321,25 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float* __restrict__ pa
     // clamped to the workspace's nsplit chunks, and records past the position's last chunk
     // (stale or never written) are masked once it has arrived -- never multiplied, so their
     // bits cannot reach the sums. The first batch always exists (chunk 0).
-    int c0 = 0, nv;
-    do {
+    // Waves 4 .. NW - 1 take no part in the first 64 chunks: they wait for the position, then all NW waves share
+    // the chunks from 64 on.
+    int c0 = 0, nv, sw = 4;  // the batch: chunks c0 + wv + sw * b
+    if (NW > 4 && wv >= 4) {
+        nv = (int)min<int64_t>(nsplit, pos / kChunk + 1);
+        c0 = 4 * B;
+        sw = NW;
+    } else {
+        nv = 1;
+    }
+    while (c0 < nv) {
         float ov[B][DPL];
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-            const int c = min(c0 + wv + 4 * b, nsplit - 1);
+            const int c = min(c0 + wv + sw * b, nsplit - 1);
 #pragma unroll
             for (int t = 0; t < DPL; ++t) ov[b][t] = base[c * stride + 2 + lane * DPL + t];
         }
-        const int cl = c0 + wv + 4 * (lane & 15);
+        const int cl = c0 + wv + sw * (lane & 15);
         const int cc = min(cl, nsplit - 1);
         float mr = base[cc * stride], lr = base[cc * stride + 1];
         __builtin_amdgcn_sched_barrier(0);
@@ -346,13 +357,14 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float* __restrict__ pa
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const float wb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), b));
-            const bool vb = c0 + wv + 4 * b < nv;  // the same in every lane
+            const bool vb = c0 + wv + sw * b < nv;  // the same in every lane
 #pragma unroll
             for (int t = 0; t < DPL; ++t) O[t] += vb ? wb * ov[b][t] : 0.f;
         }
         M = Mn;
-        c0 += 4 * B;
-    } while (c0 < nv);
+        c0 += sw * B;
+        sw = NW;
+    }
     if (lane == 0) {
         red_m[wv] = M;
         red_l[wv] = L;
@@ -362,10 +374,12 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float* __restrict__ pa
     __syncthreads();
     if (threadIdx.x < D) {
         const int d = threadIdx.x;
-        const float Mx = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));  // finite: chunk 0 exists
+        float Mx = red_m[0];  // finite: chunk 0 exists
+#pragma unroll
+        for (int w = 1; w < NW; ++w) Mx = fmaxf(Mx, red_m[w]);
         float v = 0.f, Lt = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const float f = red_m[w] == -INFINITY ? 0.f : expf(red_m[w] - Mx);
             v += f * red_o[w][d];
             Lt += f * red_l[w];
@@ -384,7 +398,14 @@ static void launch_attn(const uint16_t* q, const uint16_t* kc, const uint16_t* v
     else
         hipLaunchKernelGGL((k_attn_mfma<G, D, false>), dim3(nsplit, hk), dim3(256), 0, st, q, kc, vc, hs, pos, tmax,
                            scale, part, nsplit, QkPrep{});
-    hipLaunchKernelGGL((k_attn_merge<D>), dim3(hk * G), dim3(256), 0, st, part, pos, G, nsplit, out);
+    // The capacity decides (the position is on the device). A head's four waves walk its records 64 at a time, one
+    // round trip each: 11.0 us of merge at 512 records, 7.6 with eight waves (32 / 4 heads of 128, 32k positions: 26.5
+    // -> 23.1 us per call; 9,000 positions 12.8 -> 11.9; sixteen waves 23.3 and 13.0). Where a large cache is still
+    // short the second four waves cost 0.3 us (7.55 -> 7.83 us at 4,090 positions).
+    if (nsplit > kMergeWide)
+        hipLaunchKernelGGL((k_attn_merge<D, 8>), dim3(hk * G), dim3(512), 0, st, part, pos, G, nsplit, out);
+    else
+        hipLaunchKernelGGL((k_attn_merge<D, 4>), dim3(hk * G), dim3(256), 0, st, part, pos, G, nsplit, out);
 }
 
 static int attn_dispatch(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int64_t kv_head_stride,

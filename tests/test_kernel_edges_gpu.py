@@ -46,3 +46,28 @@ def test_attn_decode_wide_merge(Hq, Hk, D):
         ref = (w[:, None] @ vv)[:, 0]
         # one bf16 rounding (2^-9 of a value at most) and fp32 sums
         assert ((got - ref).norm() / ref.norm()).item() <= 2.0**-8, pos
+
+
+# kernel 1 rows of 2, 3 and 4 chunks per lane (a remainder in each; float32 x of four goes to the generic kernel),
+# kernel 2 with 4 to 512 (expert, chunk) pairs: part of one step, every step count, and more than 16 experts
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("H,I,group,k", [(2176, 128, 128, 1), (4096, 256, 256, 3), (4224, 128, 128, 17), (6272, 128, 128, 2),
+                                         (8192, 128, 128, 2), (256, 640, 128, 5), (4096, 512, 256, 13), (256, 1152, 128, 6),
+                                         (128, 1408, 128, 10), (128, 8192, 128, 2), (512, 384, 128, 16)])
+def test_wide_decode_layers(bits, H, I, group, k):
+    rng = np.random.default_rng(H + I + k + bits)
+    n, E = H * I, k + 1
+    pool = np.stack([O.quantize((rng.standard_normal(3 * n) * 0.02).astype(np.float32), bits, group) for _ in range(E)])
+    slots, w = rng.permutation(E)[:k], rng.random(k).astype(np.float32)
+    pt = torch.from_numpy(pool).to(DEV)
+    meta = torch.from_numpy(O.meta(slots, w)).to(DEV)
+    for xdt, tol in ((torch.bfloat16, 2.0**-8), (torch.float32, 4e-6)):  # one rounding of the result; fp32 sums
+        x = torch.from_numpy(rng.standard_normal(H).astype(np.float32)).to(xdt)
+        _, _, ref = O.moe_layer_f64(pool, slots, w, x.float().numpy(), H, I, bits, group)
+        got = kernels.moe_decode_fast(pt, meta, x.to(DEV), k, n, H, I, bits, group).double().cpu().numpy()
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        print(f"H={H} I={I} k={k} bits={bits} {xdt}: {err:.2e}")
+        assert err <= tol
+    bad = meta.clone()
+    bad[k - 1] = E  # not a slot: NaN, nothing read
+    assert torch.isnan(kernels.moe_decode_fast(pt, bad, x.to(DEV), k, n, H, I, bits, group)).all()

@@ -406,6 +406,73 @@ __global__ __launch_bounds__(64 * NW) void k_gate_up_c2(const float* __restrict_
     gate_up_rows<BITS, 64, T, QSC, XT != WISP_DT_BF16, true>(Lc, base, ok, xw, xf, act, j, r0, part[wv]);
 }
 
+// Kernel 1 for rows of more than 64 chunks (H > 2048, G = 128 * 2^i): one wave = T rows (gate and up) of one
+// expert, CPL = ceil(H / 2048) chunks of a row per lane (chunks lane, lane + 64, ...), every load issued before any use.
+// The arithmetic per chunk is k_gate_up_generic's (fp32 x, exact products); T = 2 where a
+// chunk's 32 x values, unpacked once, and their sum serve two gate and two up rows (at CPL = 4 the registers allow one row).
+// Bound by the codes' bytes and, next, VALU issue: 53.5 MB at H 4096, I 1536, k = 8, 4 bits took 17.1 us with one row per
+// single-wave workgroup and a load loop (k_gate_up_generic), 12.8 here (T = 1: 14.7, T = 4: 14.5), where a plain read of
+// the bytes takes 9.3.
+template <int BITS, int CPL, int T, int XT>
+__global__ __launch_bounds__(256) void k_gate_up_wide(const float* __restrict__ meta,
+                                                      const uint8_t* __restrict__ pool, int64_t slot_bytes,
+                                                      int nslots, const void* __restrict__ x,
+                                                      float* __restrict__ act, const Layer L) {
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = blockIdx.y, r0 = (blockIdx.x * 4 + wv) * T;
+    const float f = meta[j];
+    const int SPR = L.spr_gu;
+    int seg[CPL];
+    uint32_t xr[CPL][XWords<XT>::n];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        seg[c] = min(lane + 64 * c, SPR - 1);  // past the row: its last chunk again, added as zero
+        load_x_raw<XT>(x, seg[c], xr[c]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int slot = __builtin_amdgcn_readfirstlane(slot_from(f, nslots));
+    const uint8_t* base = pool + (int64_t)(slot >= 0 ? slot : 0) * slot_bytes;
+    const uint16_t* sc = reinterpret_cast<const uint16_t*>(base + 3 * L.nmb);
+    const int w = lane & 3;  // the lane's fp16 of its quad's group: 0 gate s, 1 gate m, 2 up s, 3 up m
+    const uint16_t* sw = sc + ((w & 1) ? 3 * (int64_t)L.NGM : 0) + ((w & 2) ? L.NGM : 0);
+    uint32_t cg[T][CPL][BITS], cu[T][CPL][BITS], sv[T][CPL];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const int r = min(r0 + t, L.I - 1);
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            const uint8_t* rp = base + (int64_t)r * L.rowb_gu + seg[c] * (4 * BITS);
+            load_chunk<BITS>(rp, cg[t][c]);
+            load_chunk<BITS>(rp + L.nmb, cu[t][c]);
+            sv[t][c] = sw[(int64_t)r * L.gpr_gu + (seg[c] >> L.gsh)];
+        }
+    }
+    float pg[T], pu[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) pg[t] = pu[t] = 0.f;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        float xf[32];
+        x_to_f32<XT>(xr[c], xf);
+        const float xs = chunk_sum_f32(xf);
+        const bool on = lane + 64 * c < SPR;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const float dg = chunk_dot_f32<BITS>(cg[t][c], xf), du = chunk_dot_f32<BITS>(cu[t][c], xf);
+            const float vg = h2f((uint16_t)quad_bcast<0>(sv[t][c])) * dg + h2f((uint16_t)quad_bcast<1>(sv[t][c])) * xs;
+            const float vu = h2f((uint16_t)quad_bcast<2>(sv[t][c])) * du + h2f((uint16_t)quad_bcast<3>(sv[t][c])) * xs;
+            pg[t] += on ? vg : 0.f;
+            pu[t] += on ? vu : 0.f;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float g = wave_sum_dpp(pg[t]), u = wave_sum_dpp(pu[t]);
+        if (lane == 0 && r0 + t < L.I) write_act(act, j, L.I, r0 + t, slot >= 0 ? silu_mul(g, u) : __builtin_nanf(""));
+    }
+}
+
 // Kernel 1 (generic): any H, G; one wave per (row, expert); x as fp32 values (exact for every x dtype).
 template <int BITS, int XT>
 __global__ __launch_bounds__(64) void k_gate_up_generic(const Layer L, const void* __restrict__ x,
@@ -777,6 +844,87 @@ __global__ __launch_bounds__(1024) void k_down_c2(const float* meta, const uint8
     down_rows<BITS, kC2I / 32, T, WSUM, QSC>(L, meta, pool, slot_bytes, nslots, k, kC2I, act, out, y, rb * RW, lds);
 }
 
+// Kernel 2 for other shapes (weighted sum, G = 128 * 2^i, k * I / 32 <= 64 NC): k_down_rows' split. A wave computes
+// one whole output row over all k experts; lane l takes the (expert, chunk) pairs l, l + 64, ..., so all lanes work
+// whatever I / 32 is and no sum crosses waves. The activations of all experts are staged once per NWV rows, piece
+// i of chunk ch at i ^ (ch & 7) (the 8 lanes of a read phase hit 8 bank groups). 26.7 MB at H 4096,
+// I 1536, k = 8, 4 bits: 10.8 us with a wave per expert (k_down: 48 of 64 lanes at work, the activations staged per 4 rows)
+// and 9.4 here; at H 5120, I 1408, k = 10 49.1 us with k_down_generic and 16.6 here; two rows per wave spill at NC = 8.
+template <int BITS, int NC, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const uint8_t* __restrict__ pool,
+                                                        int64_t slot_bytes, int nslots, int k,
+                                                        const float* __restrict__ act, void* __restrict__ out,
+                                                        const Layer L) {
+    extern __shared__ uint4 stage4[];  // k * I / 4
+    constexpr int APT = 64 * NC * 8 / (64 * NWV);
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int SPR = L.spr_dn, total = k * SPR, na = total * 8;
+    const int NB = (L.H + NWV - 1) / NWV;
+    int rb = blockIdx.x;
+    if ((NB & 7) == 0) rb = (rb & 7) * (NB >> 3) + (rb >> 3);  // each XCD one contiguous range of rows
+    const int h = rb * NWV + wv, hc = min(h, L.H - 1);
+    const float inv = __builtin_amdgcn_rcpf((float)SPR);
+    int ec[NC], sg[NC];
+    float fs[NC], fw[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int combo = min(lane + 64 * c, total - 1);
+        ec[c] = (int)(((float)combo + 0.5f) * inv);  // combo / SPR: both below 1024, the half keeps it off the edges
+        sg[c] = combo - ec[c] * SPR;
+        fs[c] = meta[ec[c]];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) fw[c] = meta[k + ec[c]];
+    const uint4* a4 = reinterpret_cast<const uint4*>(act);
+    uint4 ap[APT];
+#pragma unroll
+    for (int i = 0; i < APT; ++i) ap[i] = a4[min((int)threadIdx.x + i * 64 * NWV, na - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t cd[NC][BITS], sv[NC];
+    bool okc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int slot = slot_from(fs[c], nslots);
+        okc[c] = slot >= 0;
+        const uint8_t* base = pool + (int64_t)(okc[c] ? slot : 0) * slot_bytes;
+        const uint16_t* sc = reinterpret_cast<const uint16_t*>(base + 3 * L.nmb) + 2 * (int64_t)L.NGM;
+        const uint16_t* mn = sc + 3 * (int64_t)L.NGM;
+        const int g = sg[c] >> L.gsh;
+        load_chunk<BITS>(base + 2 * L.nmb + (int64_t)hc * L.rowb_dn + sg[c] * (4 * BITS), cd[c]);
+        const int64_t gi = (int64_t)hc * L.gpr_dn + g;
+        sv[c] = (uint32_t)sc[gi] | ((uint32_t)mn[gi] << 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the staging's waits stay behind every code load
+#pragma unroll
+    for (int i = 0; i < APT; ++i) {
+        const int idx = min((int)threadIdx.x + i * 64 * NWV, na - 1), ch = idx >> 3;
+        const uint4 a = ap[i];  // halves swapped: a plain copy could sink its load to here
+        stage4[ch * 8 + ((idx & 7) ^ (ch & 7))] = make_uint4(a.z, a.w, a.x, a.y);
+    }
+    __syncthreads();
+    float p = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int ch = min(lane + 64 * c, total - 1);
+        const bool on = lane + 64 * c < total;
+        float A[32];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint4 v = stage4[ch * 8 + (i ^ (ch & 7))];
+            A[4 * i] = __uint_as_float(v.z); A[4 * i + 1] = __uint_as_float(v.w);
+            A[4 * i + 2] = __uint_as_float(v.x); A[4 * i + 3] = __uint_as_float(v.y);
+        }
+        const float as = chunk_sum_f32(A);
+        const float d = chunk_dot_f32<BITS>(cd[c], A);
+        const float v = h2f((uint16_t)(sv[c] & 0xFFFFu)) * d + h2f((uint16_t)(sv[c] >> 16)) * as;
+        p = __builtin_fmaf(fw[c], !on ? 0.f : okc[c] ? v : __builtin_nanf(""), p);
+        __builtin_amdgcn_sched_barrier(0);  // one chunk's activations in registers at a time
+    }
+    const float tot = wave_sum_dpp(p);
+    if (lane == 0 && h < L.H) store_out(out, L.odt, h, tot);
+}
+
 // Kernel 2 (generic): any I, G and k; one workgroup of min(k, 16) waves per
 // output row, wave w takes experts w, w + 16, ...; the k expert sums meet in
 // LDS (dynamic, k floats) and are combined in expert order.
@@ -896,6 +1044,17 @@ static void launch_gu(const Layer& L, const void* x, float* act, hipStream_t st)
 
 template <int BITS, int XT>
 static int gate_up_bits(const Layer& L, const void* x, float* act, hipStream_t st) {
+    // more than 64 chunks per row. Four chunks of a float32 x per lane take 170 registers: the generic kernel's one row per wave is as fast there
+    if (L.spr_gu > 64 && L.spr_gu <= (XT == WISP_DT_F32 ? 192 : 256) && L.gsh >= 2) {
+#define WISP_GW(C, T)                                                                                               \
+    hipLaunchKernelGGL((k_gate_up_wide<BITS, C, T, XT>), dim3((L.I + 4 * T - 1) / (4 * T), L.k), dim3(256), 0, st,  \
+                       L.meta, L.pool, L.slot_bytes, L.nslots, x, act, L)
+        if (L.spr_gu <= 128) WISP_GW(2, 2);
+        else if (L.spr_gu <= 192) WISP_GW(3, 2);
+        else WISP_GW(4, 1);
+#undef WISP_GW
+        return check_launch("k_gate_up_wide");
+    }
     if (L.spr_gu > 64 || L.gsh < 0) {
         hipLaunchKernelGGL((k_gate_up_generic<BITS, XT>), dim3(L.I, L.k), dim3(64), 0, st, L, x, act);
         return check_launch("k_gate_up_generic");
@@ -952,7 +1111,32 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
     // the fast path has one wave per expert (k <= 16) and stages k*I activation
     // values in LDS: keep the whole LDS within 64 KB
     const bool tuned = L.spr_dn == 24 && L.gsh >= 2;
-    if (L.k > 16 || L.spr_dn > 64 || L.gsh < 0 || dn_lds_bytes(L, tuned ? tuning().dn_iters : 4) > 65536) {
+    const bool waves = L.k <= 16 && L.spr_dn <= 64 && L.gsh >= 0 &&
+                       dn_lds_bytes(L, tuned ? tuning().dn_iters : 4) <= 65536;  // one wave per expert: k_down
+    const int64_t pairs = (int64_t)L.k * L.spr_dn;
+    // k_down_wide keeps every lane at work and needs no particular k; k_down stages a quarter of the activations per
+    // row and stays where it can run (`waves`) with few output rows and many pairs: layers of 2,048 rows at k = 8 took
+    // 10.05 us with it against 10.35 (I 1024) and 11.6 against 12.0 (I 1408, k = 6), and 8.8 against 8.0 (I 1024, k = 5),
+    // 13.5 against 11.2 (3,072 rows, I 1152, k = 4) the other way. I = 768 keeps its tuned forms.
+    if (WSUM && L.gsh >= 2 && pairs <= 512 && !(waves && (tuned || (L.H <= 2048 && pairs > 192)))) {
+        const bool n8 = L.H >= 4096;  // eight rows per staged activation once that still leaves two workgroups per CU
+#define WISP_DW(C, NWV)                                                                                               \
+    hipLaunchKernelGGL((k_down_wide<BITS, C, NWV>), dim3((L.H + NWV - 1) / NWV), dim3(64 * NWV), (size_t)pairs * 128, \
+                       st, L.meta, L.pool, L.slot_bytes, L.nslots, L.k, act, out, L)
+        if (pairs <= 64) WISP_DW(1, 4);
+        else if (pairs <= 128) WISP_DW(2, 4);
+        else if (pairs <= 192 && n8) WISP_DW(3, 8);
+        else if (pairs <= 192) WISP_DW(3, 4);
+        else if (pairs <= 256 && n8) WISP_DW(4, 8);
+        else if (pairs <= 256) WISP_DW(4, 4);
+        else if (pairs <= 384 && n8) WISP_DW(6, 8);
+        else if (pairs <= 384) WISP_DW(6, 4);
+        else if (n8) WISP_DW(8, 8);
+        else WISP_DW(8, 4);
+#undef WISP_DW
+        return check_launch("k_down_wide");
+    }
+    if (!waves) {
         const int nw = L.k < 16 ? L.k : 16;
         hipLaunchKernelGGL((k_down_generic<BITS, WSUM>), dim3(L.H), dim3(64 * nw), WSUM ? sizeof(float) * L.k : 0, st,
                            L, act, out, y);

@@ -201,6 +201,19 @@ int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, co
                      int k, int64_t H, int64_t I, int bits, int64_t group, void* ws, uint16_t* out, float* acc,
                      void* stream);
 
+/* wisp_moe_prefill planned on the GPU: groups, tok, w and back are formed by one kernel from the routing in device
+ * memory (no host synchronisation; capturable). sel: [T][k] expert ids, contiguous, int32 or int64 (sel_bytes 4 or 8);
+ * rw: [T][k] routing weights of rw_dtype (WISP_DT_*); slot_of: HOST int32 [n_ids], read before the call returns: the
+ * slot of expert id i, or INT32_MIN for an expert that this call does not run (its pairs, and those of ids outside
+ * [0, n_ids), add nothing); at least one present, n_ids <= 512. max_pairs: at least the number of pairs of present
+ * experts, T*k if unknown (with fewer the outputs are undefined; nothing is accessed out of bounds). ws:
+ * wisp_prefill_routed_ws_bytes(T, k, max_pairs, n_ids, H, I), 256-byte aligned. Everything else as wisp_moe_prefill. */
+int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t max_pairs, int64_t n_ids, int64_t H, int64_t I);
+int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const void* sel, int sel_bytes,
+                            const void* rw, int rw_dtype, const int32_t* slot_of, int n_ids, int64_t max_pairs,
+                            const uint16_t* x, int T, int k, int64_t H, int64_t I, int bits, int64_t group, void* ws,
+                            uint16_t* out, float* acc, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Expert cache bookkeeping (host only, no device calls). Keys are
  * layer*n_experts + expert; slots [0, n_static) are the static region.
@@ -267,6 +280,10 @@ int wisp_cache_issue(void* cache, const int64_t* keys, const int64_t* slots, int
 int wisp_cache_sync_compute(void* cache, void* compute);
 /* cache.py:87-91 (ensure): residency, copies, ordering, in one call. */
 int wisp_cache_ensure(void* cache, const int64_t* keys, int64_t n, int64_t* slots, void* compute);
+/* wisp_cache_ensure of keys[0, chunk), keys[chunk, 2*chunk), ... in turn (the same bookkeeping as that many calls),
+ * stopping at the first that fails. A later chunk may reuse an earlier chunk's slot, except with the lru policy and no
+ * more keys than dynamic slots: every slot of this call is then younger than the one a miss evicts. */
+int wisp_cache_ensure_chunks(void* cache, const int64_t* keys, int64_t n, int64_t chunk, int64_t* slots, void* compute);
 /* One layer's host step of the graph decoder (graphdec.py:216-231): ensure the
  * k routed keys, write [slots | weights] into meta_host (pinned float32 [2k])
  * and copy it to meta_dev on `compute`. slots (may be NULL) receives the slots. */

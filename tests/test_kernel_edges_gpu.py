@@ -1,10 +1,15 @@
 """The kernels' tile edges, remainders and dispatch rules against the CPU oracle."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import oracle as O
 from wisp import kernels, quant
+from wisp.cache import ExpertCache
+from wisp.moe import PagedMoEBlock, Runtime, route
+from wisp.store import ExpertStore
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -71,3 +76,103 @@ def test_wide_decode_layers(bits, H, I, group, k):
     bad = meta.clone()
     bad[k - 1] = E  # not a slot: NaN, nothing read
     assert torch.isnan(kernels.moe_decode_fast(pt, bad, x.to(DEV), k, n, H, I, bits, group)).all()
+
+
+def _routing(gen, T, E, k):
+    p = torch.randn((T, E), generator=gen, device=DEV).softmax(-1)
+    rw, sel = p.topk(k, -1)
+    return sel, rw.to(torch.bfloat16)
+
+
+# the plan formed on the GPU against the host's, bit for bit: one token, runs that are not whole waves, a hot expert
+# (more matches in a wave's run than its list holds), every chunk size, the largest table, k = 32 (the wide combine)
+@pytest.mark.parametrize("E,k,T,bits", [(6, 2, 1, 4), (6, 2, 17, 3), (4, 2, 900, 4), (300, 8, 50, 2), (512, 4, 40, 4),
+                                        (40, 32, 33, 4), (3, 1, 9000, 4), (5, 3, 333, 3)])
+@pytest.mark.parametrize("mode", ["all", "part", "twice", "outside"])
+def test_prefill_plan_on_the_gpu_equals_the_hosts(E, k, T, bits, mode):
+    H, I, n = 256, 128, 256 * 128
+    rng = np.random.default_rng(E + T)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(6)])).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(E * 31 + T)
+    x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
+    sel, rw = _routing(gen, T, E, k)
+    slots = {e: e % 6 for e in range(E)}
+    if mode == "part":  # some experts absent, one with no such slot (its tokens become NaN)
+        slots = {e: e % 6 for e in range(0, E, 2)}
+        slots[max(slots)] = 77
+    if mode == "twice":  # an expert chosen twice by one token
+        sel[:, -1] = sel[:, 0]
+    if mode == "outside":  # ids that no table holds
+        sel[::3, 0], sel[1::3, -1] = -1, 1 << 40
+    for w in (rw, rw.float(), rw.half()):
+        got = kernels.moe_prefill(pool, slots, x, sel, w, n, H, I, bits)
+        want = kernels.moe_prefill(pool, slots, x, sel.cpu(), w, n, H, I, bits)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    s32 = sel.clamp(max=1 << 20).int()
+    acc, ref = torch.full((T, H), 0.25, device=DEV), torch.full((T, H), 0.25, device=DEV)
+    kernels.moe_prefill(pool, slots, x, s32, rw, n, H, I, bits, acc=acc)
+    kernels.moe_prefill(pool, slots, x, s32.cpu(), rw, n, H, I, bits, acc=ref)
+    assert torch.equal(acc.view(torch.int32), ref.view(torch.int32))
+
+
+def test_prefill_under_graph_capture_follows_the_routing():
+    E, k, T, H, I, bits, n = 8, 2, 70, 256, 128, 4, 256 * 128
+    rng = np.random.default_rng(5)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(E)])).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
+    sel, rw = _routing(gen, T, E, k)
+    slots = {e: e for e in range(E)}
+    kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits)
+    for _ in range(4):
+        s2, r2 = _routing(gen, T, E, k)
+        sel.copy_(s2)
+        rw.copy_(r2)
+        g.replay()
+        torch.cuda.synchronize()
+        want = kernels.moe_prefill(pool, slots, x, s2.cpu(), r2, n, H, I, bits)
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("nslots,n_static,policy", [(12, 0, "lru"), (16, 3, "lru"), (9, 0, "lru"), (12, 0, "wsa")])
+def test_block_runs_all_experts_at_once_where_the_cache_holds_them(nslots, n_static, policy):
+    """A paged block's prefill pages in chunks of rt.chunk experts whatever the cache holds: the bookkeeping equals the
+    chunk-by-chunk calls, and the output the oracle's, with and without room for all routed experts."""
+    E, k, T, H, I, bits, n = 12, 4, 40, 256, 128, 4, 256 * 128
+    gen = torch.Generator(device=DEV).manual_seed(nslots + n_static)
+    store = ExpertStore(1, E, n, bits, 128)
+    store.fill(((e, torch.randn((3, n), generator=gen, device=DEV) * 0.05) for e in range(E)))
+    pre = list(range(n_static))
+    caches = [ExpertCache(store, nslots, policy=policy, n_static=n_static, preload_keys=pre or None) for _ in range(2)]
+    rt = Runtime(store, caches[0], chunk=5)
+    gate = torch.nn.Linear(H, E, bias=False, device=DEV, dtype=torch.bfloat16)
+    cfg = SimpleNamespace(hidden_size=H, moe_intermediate_size=I, num_experts=E, num_experts_per_tok=k,
+                          norm_topk_prob=True)
+    block = PagedMoEBlock(gate, 0, rt, cfg)
+    for step in range(3):
+        x = torch.randn((1, T, H), generator=gen, device=DEV).to(torch.bfloat16)
+        with torch.no_grad():
+            y = block(x)
+            logits = gate(x[0])
+        y = y[0] if isinstance(y, tuple) else y
+        sel, rw = route(logits, k, True, x.dtype)
+        keys = torch.unique(sel.cpu()).tolist()
+        want = []
+        for i in range(0, len(keys), 5):
+            want += list(zip(keys[i : i + 5], caches[1].ensure(keys[i : i + 5])))
+        a, b = caches[0].core, caches[1].core
+        assert a.stats == b.stats
+        assert [a.lookup(e) for e in range(E)] == [b.lookup(e) for e in range(E)]
+        xb = x[0].view(torch.int16).cpu().numpy().view(np.uint16)
+        ref = O.moe_prefill_f64(store.host.numpy(), {e: e for e in range(E)}, xb, sel.cpu().numpy(),
+                                rw.float().cpu().numpy(), H, I, bits)
+        err = np.linalg.norm(y[0].double().cpu().numpy() - ref) / np.linalg.norm(ref)
+        assert err <= 2.0**-8, (step, err)
+    for c in caches:
+        c.free()

@@ -1327,6 +1327,18 @@ extern "C" int wisp_cache_ensure(void* h, const int64_t* keys, int64_t n, int64_
     return sync_compute(c, (hipStream_t)compute);
 }
 
+// moe.py:120-129: a chunk of a prefill's experts after another
+extern "C" int wisp_cache_ensure_chunks(void* h, const int64_t* keys, int64_t n, int64_t chunk, int64_t* slots,
+                                        void* compute) {
+    clear_error();
+    if (n < 0 || chunk < 1 || (n && (!keys || !slots))) return fail_inval("bad ensure_chunks args");
+    for (int64_t i = 0; i < n; i += chunk) {
+        const int rc = wisp_cache_ensure(h, keys + i, std::min(chunk, n - i), slots + i, compute);
+        if (rc) return rc;
+    }
+    return WISP_OK;
+}
+
 // graphdec.py:216-231 for one layer: slots = ensure(keys); meta_host = [slots |
 // weights] (pinned, float32 [2k]); meta_dev <- meta_host on the compute stream,
 // ordered after the expert copies. Returns the slots in `slots` (may be NULL).

@@ -42,6 +42,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "wisp_device.hpp"
@@ -913,8 +914,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // s = sum_j y[back[t*k + j]][h], j in ascending expert id (back = -1: no pair in
 // this call); out[t][h] = bf16(s), or acc[t][h] += s when acc is given.
 // A thread takes 4 consecutive h of one token; its up to KMAX y rows are all
-// requested before the ordered sum (k <= KMAX; H % 4 == 0).
-template <int KMAX>
+// requested before the ordered sum (k <= KMAX; H % 4 == 0). SORT: back[t*k + j] is the pair of
+// the token's j-th expert as routed (k_pf_plan); ascending pairs are ascending experts.
+template <int KMAX, bool SORT>
 __global__ __launch_bounds__(256) void k_pf_combine(const float* __restrict__ y, const int32_t* __restrict__ back,
                                                     int T, int k, int H, int P, uint16_t* __restrict__ out,
                                                     float* __restrict__ acc) {
@@ -928,6 +930,23 @@ __global__ __launch_bounds__(256) void k_pf_combine(const float* __restrict__ y,
     int pj[KMAX];
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) pj[j] = back[t * k + min(j, k - 1)];
+    if constexpr (SORT) {  // odd-even merge sort; the repeated pairs past k sort last and are skipped
+#pragma unroll
+        for (int j = 0; j < KMAX; ++j) pj[j] = j < k ? pj[j] : INT32_MAX;
+#pragma unroll
+        for (int p = 1; p < KMAX; p <<= 1)
+#pragma unroll
+            for (int q = p; q >= 1; q >>= 1)
+#pragma unroll
+                for (int j = q % p; j + q < KMAX; j += 2 * q)
+#pragma unroll
+                    for (int i = 0; i < q; ++i)
+                        if (i + j + q < KMAX && (i + j) / (2 * p) == (i + j + q) / (2 * p)) {
+                            const int lo = min(pj[i + j], pj[i + j + q]), hi = max(pj[i + j], pj[i + j + q]);
+                            pj[i + j] = lo;
+                            pj[i + j + q] = hi;
+                        }
+    }
     __builtin_amdgcn_sched_barrier(0);
     float4 v[KMAX];
 #pragma unroll
@@ -954,6 +973,149 @@ __global__ __launch_bounds__(256) void k_pf_combine(const float* __restrict__ y,
     } else {
         *reinterpret_cast<uint2*>(out + i) = make_uint2(pack_bf16x2(s.x, s.y), pack_bf16x2(s.z, s.w));
     }
+}
+
+// ===========================================================================
+// The routing plan on the GPU: tok, w, back and the work items of wisp_moe_prefill from sel [T, k] and rw [T, k], so
+// a prefill needs neither the routing on the host nor an upload. One workgroup per expert id of the table and one
+// more; each reads all T*k pairs and counts those of its expert and of the ones before it (no order between workgroups,
+// nothing to clear), then lists its own pairs in token order: a wave takes a contiguous run of the pairs and places
+// its matches by ballots (more than kPlanList of one expert in a run are read again). The last workgroup marks the pairs of absent experts and writes the
+// work items, each expert's pairs split evenly (a multiple of 16) into ceil(count / chunk) items, items of more token
+// tiles first; entries past the last item get no pairs. Bound by the reads of sel (every workgroup
+// reads it, from L2): and by the ballots' issue: 5.1 us for 64 tokens, 18 for
+// 4,096 (8 experts each); the grouping in numpy and its uploads took about 100 and 1,600 us, after a wait for the GPU.
+// ===========================================================================
+constexpr int kPlanIds = 512, kPlanWaves = 16, kPlanList = 256;
+constexpr int32_t kPlanAbsent = INT32_MIN;
+struct PlanTable {
+    int32_t slot[kPlanIds];  // slot of each expert id, kPlanAbsent where the call does not run it
+};
+struct PlanOut {
+    int32_t* groups;  // [U][3]
+    int32_t* tok;     // [P]
+    float* w;         // [P]
+    int32_t* back;    // [T][k]
+    int U, P, chunk;
+};
+
+__device__ __forceinline__ float plan_w(const void* rw, int rdt, int64_t i) {
+    if (rdt == WISP_DT_BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(rw)[i]);
+    if (rdt == WISP_DT_F16) return h2f(reinterpret_cast<const uint16_t*>(rw)[i]);
+    return reinterpret_cast<const float*>(rw)[i];
+}
+
+template <typename ST>
+__global__ __launch_bounds__(64 * kPlanWaves) void k_pf_plan(const ST* __restrict__ sel, const void* __restrict__ rw,
+                                                             int rdt, int T, int k, int nids, const PlanTable tb,
+                                                             const PlanOut po) {
+    __shared__ int hist[kPlanIds + 1], slots[kPlanIds + 1], wmine[kPlanWaves], wless[kPlanWaves], list[kPlanWaves][kPlanList];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x;
+    if (b < nids && tb.slot[b] == kPlanAbsent) return;  // the whole workgroup
+    for (int i = tid; i <= nids; i += 64 * kPlanWaves) {
+        hist[i] = 0;
+        slots[i] = i < nids ? tb.slot[i] : kPlanAbsent;
+    }
+    __syncthreads();
+    const int n = T * k, per = ((n + kPlanWaves - 1) / kPlanWaves + 63) & ~63;
+    const int i0 = min(n, wv * per), i1 = min(n, i0 + per);
+    // The wave's pairs, 64 * B at a time with every load of a batch in flight: f(pair, bin, within the run); the
+    // bin is nids for an expert the call does not run.
+    constexpr int B = 8;
+    auto each = [&](auto f) {
+        for (int i = i0; i < i1; i += 64 * B) {
+            ST id[B];
+#pragma unroll
+            for (int u = 0; u < B; ++u) id[u] = sel[min(i + 64 * u + lane, n - 1)];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                if (i + 64 * u >= i1) break;
+                const int e = id[u] >= 0 && id[u] < nids ? (int)id[u] : nids;
+                f(i + 64 * u + lane, slots[e] != kPlanAbsent ? e : nids, i + 64 * u + lane < i1);
+            }
+        }
+    };
+    // First all pairs are counted, the matches also listed; then each wave places its own.
+    int mine = 0, less = 0;
+    each([&](int p, int bin, bool in) {
+        const uint64_t m = __ballot(in && bin == b);
+        const int at = mine + __popcll(m & ((1ull << lane) - 1));
+        if (in && bin == b && at < kPlanList) list[wv][at] = p;
+        mine += __popcll(m);
+        less += __popcll(__ballot(in && bin < b));
+        if (b == nids && in) atomicAdd(&hist[bin], 1);  // only the items need every expert's count
+    });
+    if (lane == 0) {
+        wmine[wv] = mine;
+        wless[wv] = less;
+    }
+    __syncthreads();
+    int base = 0;  // this wave's first pair of the expert
+    for (int i = 0; i < kPlanWaves; ++i) base += wless[i] + (i < wv ? wmine[i] : 0);
+    auto place = [&](int p, int at) {
+        const bool room = b < nids && at < po.P;
+        po.back[p] = b == nids ? -1 : room ? at : po.P;
+        if (room) {
+            po.tok[at] = p / k;
+            po.w[at] = plan_w(rw, rdt, p);
+        }
+    };
+    if (mine <= kPlanList) {
+        for (int i = lane; i < mine; i += 64) place(list[wv][i], base + i);
+    } else {
+        each([&](int p, int bin, bool in) {
+            const uint64_t m = __ballot(in && bin == b);
+            if (in && bin == b) place(p, base + __popcll(m & ((1ull << lane) - 1)));
+            base += __popcll(m);
+        });
+    }
+    if (b < nids) return;
+    // The work items, one thread per expert. Their order among items of equal tiles is left to the atomics: it does not
+    // reach any result.
+    __shared__ int tiles[9], first_u[9];  // items of t tiles, and the first free place for the next
+    if (tid < 9) tiles[tid] = 0;
+    __syncthreads();
+    int c = 0, nf = 0, full = 0, last = 0, incl = 0;
+    if (tid < kPlanIds) {
+        c = tid < nids ? hist[tid] : 0;  // (an absent expert's pairs are counted at nids)
+        if (c) {
+            const int ni = (c + po.chunk - 1) / po.chunk;
+            nf = ni - 1;
+            full = ((c + ni - 1) / ni + 15) / 16;  // 16-pair tiles of every item but the last
+            last = (c - nf * 16 * full + 15) / 16;
+            if (nf) atomicAdd(&tiles[full], nf);
+            atomicAdd(&tiles[last], 1);
+        }
+        incl = c;  // pairs up to and with this expert's, within the wave
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
+        }
+        if (lane == 63) wmine[wv] = incl;
+    }
+    __syncthreads();
+    int used = 0;
+    for (int t = 8; t >= 1; --t) {
+        if (tid == 0) first_u[t] = used;
+        used += tiles[t];
+    }
+    __syncthreads();
+    if (c) {
+        int first = incl - c;
+        for (int i = 0; i < wv; ++i) first += wmine[i];
+        const int uf = nf ? atomicAdd(&first_u[full], nf) : 0, ul = atomicAdd(&first_u[last], 1);
+        for (int i = 0; i <= nf; ++i) {
+            const int u = i < nf ? uf + i : ul, p0 = first + i * 16 * full;
+            const int cnt = i < nf ? 16 * full : c - nf * 16 * full;
+            if (u < po.U) {
+                po.groups[3 * u] = slots[tid];
+                po.groups[3 * u + 1] = min(p0, po.P);
+                po.groups[3 * u + 2] = max(0, min(cnt, po.P - p0));
+            }
+        }
+    }
+    for (int u = used + tid; u < po.U; u += 64 * kPlanWaves)  // past the last item: no pairs
+        po.groups[3 * u] = po.groups[3 * u + 1] = po.groups[3 * u + 2] = 0;
 }
 
 // MT (16-token tiles per wave and pass) from the largest group; Z workgroups
@@ -1020,6 +1182,60 @@ extern "C" int64_t wisp_prefill_ws_bytes(int64_t pairs, int64_t H, int64_t I) {
     return (pairs * I * 2 + 255) / 256 * 256 + pairs * H * 4;
 }
 
+// The checks and launches shared by the two entries; groups (with max_group), tok, w, back and the work space are set.
+static int prefill_check(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const uint16_t* x, int T, int k,
+                         int64_t pairs, int64_t H, int64_t I, int bits, int64_t group, const void* ws, const uint16_t* out,
+                         const float* acc) {
+    if (!(bits == 4 || bits == 3 || bits == 2)) return fail_inval("bits must be 4, 3 or 2");
+    if (group != 128) return fail_inval("the grouped prefill needs group 128 (one quant group per K step)");
+    if (H % 256 || I % 128 || H > (1 << 16) || I > (1 << 16))
+        return fail_inval("H a multiple of 256 and I of 128, both <= 65536");
+    if (T < 1 || k < 1 || k > 32 || pairs < 1 || pairs > (int64_t)T * k)
+        return fail_inval("need 1 <= k <= 32, 1 <= pairs <= T*k and at least one group");
+    if (nslots < 1 || nslots > (1 << 24)) return fail_inval("nslots out of range");
+    if (slot_bytes < wisp_expert_nbytes(H * I, bits, group)) return fail_inval("slot_bytes < expert size");
+    if (!aligned(pool, 16) || slot_bytes % 16 || !aligned(x, 16) || !aligned(ws, 256) || (out && !aligned(out, 8)) ||
+        (acc && !aligned(acc, 16))) {
+        set_error("pool, x, ws, out and acc must be 16/16/256/8/16-byte aligned, slot_bytes a multiple of 16");
+        return WISP_EALIGN;
+    }
+    return WISP_OK;
+}
+
+static int prefill_launch(Prefill& F, const uint8_t* pool, int64_t slot_bytes, int64_t nslots, int ngroups,
+                          int max_group, const int32_t* back, bool sorted, int64_t pairs, const uint16_t* x, int T, int k,
+                          int64_t H, int64_t I, int bits, void* ws, uint16_t* out, float* acc, hipStream_t st) {
+    const int64_t n = H * I;
+    F.pool = pool;
+    F.slot_bytes = slot_bytes;
+    F.nmb = n * bits / 8;
+    F.nslots = (int)nslots;
+    F.H = (int)H;
+    F.I = (int)I;
+    F.NGM = (int)(n / 128);
+    F.P = (int)pairs;
+    F.T = T;
+    F.x = x;
+    F.act = static_cast<uint16_t*>(ws);
+    F.y = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + (pairs * I * 2 + 255) / 256 * 256);
+    F.gy = F.gz = 1;  // set per launch for the LDS-DMA kernels
+    switch (bits) {
+    case 4: launch_pf<4>(F, ngroups, max_group, st); break;
+    case 3: launch_pf<3>(F, ngroups, max_group, st); break;
+    default: launch_pf<2>(F, ngroups, max_group, st); break;
+    }
+    const unsigned nblk = (unsigned)(((int64_t)T * H / 4 + 255) / 256);
+#define WISP_CB(K, S)                                                                                                 \
+    hipLaunchKernelGGL((k_pf_combine<K, S>), dim3(nblk), dim3(256), 0, st, (const float*)F.y, back, T, k, (int)H,     \
+                       (int)pairs, out, acc)
+    if (sorted && k <= 8) WISP_CB(8, false);
+    else if (sorted) WISP_CB(32, false);
+    else if (k <= 8) WISP_CB(8, true);
+    else WISP_CB(32, true);
+#undef WISP_CB
+    return check_launch("k_pf");
+}
+
 // moe.py:131-151 (grouped: one launch per GEMM for all routed experts)
 extern "C" int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const int32_t* groups,
                                 int ngroups, int max_group, const int32_t* tok, const float* w, const int32_t* back, int64_t pairs,
@@ -1027,50 +1243,82 @@ extern "C" int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t
                                 void* ws, uint16_t* out, float* acc, void* stream) {
     clear_error();
     if (!pool || !groups || !tok || !w || !back || !x || !ws || (!out && !acc)) return fail_inval("null pointer");
-    if (!(bits == 4 || bits == 3 || bits == 2)) return fail_inval("bits must be 4, 3 or 2");
-    if (group != 128) return fail_inval("the grouped prefill needs group 128 (one quant group per K step)");
-    if (H % 256 || I % 128 || H > (1 << 16) || I > (1 << 16))
-        return fail_inval("H a multiple of 256 and I of 128, both <= 65536");
-    if (T < 1 || k < 1 || k > 32 || ngroups < 1 || pairs < 1 || pairs > (int64_t)T * k)
-        return fail_inval("need 1 <= k <= 32, 1 <= pairs <= T*k and at least one group");
-    if (nslots < 1 || nslots > (1 << 24)) return fail_inval("nslots out of range");
-    const int64_t n = H * I;
-    if (slot_bytes < wisp_expert_nbytes(n, bits, group)) return fail_inval("slot_bytes < expert size");
-    if (!aligned(pool, 16) || slot_bytes % 16 || !aligned(x, 16) || !aligned(ws, 256) || (out && !aligned(out, 8)) ||
-        (acc && !aligned(acc, 16))) {
-        set_error("pool, x, ws, out and acc must be 16/16/256/8/16-byte aligned, slot_bytes a multiple of 16");
-        return WISP_EALIGN;
-    }
+    if (ngroups < 1) return fail_inval("need 1 <= k <= 32, 1 <= pairs <= T*k and at least one group");
+    const int rc = prefill_check(pool, slot_bytes, nslots, x, T, k, pairs, H, I, bits, group, ws, out, acc);
+    if (rc) return rc;
     Prefill F;
-    F.pool = pool;
-    F.slot_bytes = slot_bytes;
-    F.nmb = n * bits / 8;
-    F.nslots = (int)nslots;
-    F.H = (int)H;
-    F.I = (int)I;
-    F.NGM = (int)(n / group);
-    F.P = (int)pairs;
-    F.T = T;
     F.groups = groups;
     F.tok = tok;
     F.w = w;
-    F.x = x;
-    F.act = static_cast<uint16_t*>(ws);
-    F.y = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + (pairs * I * 2 + 255) / 256 * 256);
-    F.gy = F.gz = 1;  // set per launch for the LDS-DMA kernels
-    hipStream_t st = (hipStream_t)stream;
     max_group = std::max(1, std::min(max_group, T));  // a launch-shape hint; any value is correct
-    switch (bits) {
-    case 4: launch_pf<4>(F, ngroups, max_group, st); break;
-    case 3: launch_pf<3>(F, ngroups, max_group, st); break;
-    default: launch_pf<2>(F, ngroups, max_group, st); break;
+    return prefill_launch(F, pool, slot_bytes, nslots, ngroups, max_group, back, true, pairs, x, T, k, H, I, bits, ws, out,
+                          acc, (hipStream_t)stream);
+}
+
+// Work items a plan of `pairs` pairs over `present` experts can need: one per expert that has any, and one more for
+// every full chunk.
+static int64_t plan_items(int64_t pairs, int64_t present, int chunk) {
+    return std::max<int64_t>(1, std::min(pairs, present + pairs / chunk));
+}
+// Pairs per work item: the smallest of 16, 32, 64 and 128 that the mean of an expert's pairs plus two of its
+// (Poisson) deviations fits. Fewer tiles per pass leave more workgroups per CU, and items that are split read their
+// expert's rows twice. The outputs do not depend on it.
+static int plan_chunk(int64_t pairs, int64_t present) {
+    const double mean = (double)pairs / (double)std::max<int64_t>(1, present), most = mean + 2 * std::sqrt(mean);
+    return most <= 16 ? 16 : most <= 32 ? 32 : most <= 64 ? 64 : 128;
+}
+static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
+
+extern "C" int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t max_pairs, int64_t n_ids, int64_t H, int64_t I) {
+    if (T < 1 || k < 1 || max_pairs < 1 || max_pairs > T * k || n_ids < 1 || n_ids > kPlanIds || H < 1 || I < 1) return -1;
+    return up256(12 * plan_items(max_pairs, n_ids, 16)) + up256(8 * max_pairs) + up256(4 * T * k) +
+           wisp_prefill_ws_bytes(max_pairs, H, I);
+}
+
+// moe.py:82-151: the grouping of the (token, expert) pairs and wisp_moe_prefill, from the routing in device memory
+extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const void* sel,
+                                       int sel_bytes, const void* rw, int rw_dtype, const int32_t* slot_of, int n_ids,
+                                       int64_t max_pairs, const uint16_t* x, int T, int k, int64_t H, int64_t I, int bits,
+                                       int64_t group, void* ws, uint16_t* out, float* acc, void* stream) {
+    clear_error();
+    if (!pool || !sel || !rw || !slot_of || !x || !ws || (!out && !acc)) return fail_inval("null pointer");
+    if (sel_bytes != 4 && sel_bytes != 8) return fail_inval("sel must be int32 or int64");
+    if (rw_dtype != WISP_DT_BF16 && rw_dtype != WISP_DT_F16 && rw_dtype != WISP_DT_F32)
+        return fail_inval("rw_dtype must be WISP_DT_BF16, WISP_DT_F16 or WISP_DT_F32");
+    if (n_ids < 1 || n_ids > kPlanIds) return fail_inval("n_ids must be in [1, 512]");
+    if ((int64_t)T * k >= (int64_t)1 << 31) return fail_inval("T*k must be below 2^31");
+    const int rc = prefill_check(pool, slot_bytes, nslots, x, T, k, max_pairs, H, I, bits, group, ws, out, acc);
+    if (rc) return rc;
+    PlanTable tb;
+    int64_t present = 0;
+    for (int i = 0; i < kPlanIds; ++i) {
+        tb.slot[i] = i < n_ids ? slot_of[i] : kPlanAbsent;
+        present += tb.slot[i] != kPlanAbsent;
     }
-    const unsigned nblk = (unsigned)(((int64_t)T * H / 4 + 255) / 256);
-    if (k <= 8)
-        hipLaunchKernelGGL(k_pf_combine<8>, dim3(nblk), dim3(256), 0, st, (const float*)F.y, back, T, k, (int)H,
-                           (int)pairs, out, acc);
+    if (!present) return fail_inval("no expert in slot_of");
+    PlanOut po;
+    po.chunk = plan_chunk(max_pairs, present);
+    po.U = (int)plan_items(max_pairs, present, po.chunk);
+    po.P = (int)max_pairs;
+    uint8_t* at = static_cast<uint8_t*>(ws);
+    po.groups = reinterpret_cast<int32_t*>(at);
+    at += up256(12 * plan_items(max_pairs, n_ids, 16));
+    po.tok = reinterpret_cast<int32_t*>(at);
+    po.w = reinterpret_cast<float*>(at + 4 * max_pairs);
+    at += up256(8 * max_pairs);
+    po.back = reinterpret_cast<int32_t*>(at);
+    at += up256(4 * (int64_t)T * k);
+    hipStream_t st = (hipStream_t)stream;
+    if (sel_bytes == 8)
+        hipLaunchKernelGGL(k_pf_plan<int64_t>, dim3(n_ids + 1), dim3(64 * kPlanWaves), 0, st, (const int64_t*)sel, rw,
+                           rw_dtype, T, k, n_ids, tb, po);
     else
-        hipLaunchKernelGGL(k_pf_combine<32>, dim3(nblk), dim3(256), 0, st, (const float*)F.y, back, T, k, (int)H,
-                           (int)pairs, out, acc);
-    return check_launch("k_pf");
+        hipLaunchKernelGGL(k_pf_plan<int32_t>, dim3(n_ids + 1), dim3(64 * kPlanWaves), 0, st, (const int32_t*)sel, rw,
+                           rw_dtype, T, k, n_ids, tb, po);
+    Prefill F;
+    F.groups = po.groups;
+    F.tok = po.tok;
+    F.w = po.w;
+    return prefill_launch(F, pool, slot_bytes, nslots, po.U, std::min(po.chunk, T), po.back, false, max_pairs, x, T, k, H, I,
+                          bits, at, out, acc, st);
 }

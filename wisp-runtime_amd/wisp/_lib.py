@@ -47,6 +47,9 @@ SIGNATURES = {
     "wisp_prefill_ws_bytes": (_i64, [_i64, _i64, _i64]),
     "wisp_moe_prefill": (_i32, [_vp, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _vp, _i32, _i32, _i64, _i64,
                                 _i32, _i64, _vp, _vp, _vp, _vp]),
+    "wisp_prefill_routed_ws_bytes": (_i64, [_i64, _i32, _i64, _i64, _i64, _i64]),
+    "wisp_moe_prefill_routed": (_i32, [_vp, _i64, _i64, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _vp, _i32, _i32, _i64, _i64,
+                                       _i32, _i64, _vp, _vp, _vp, _vp]),
     "wisp_mxfp4_to_bf16": (_i32, [_vp, _vp, _i64, _vp, _vp]),
     "wisp_dl_gemv": (_i32, [_vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp,
                             _vp, _vp]),
@@ -81,6 +84,7 @@ SIGNATURES = {
     "wisp_cache_issue": (_i32, [_vp, _vp, _vp, _i64, _vp]),
     "wisp_cache_sync_compute": (_i32, [_vp, _vp]),
     "wisp_cache_ensure": (_i32, [_vp, _vp, _i64, _vp, _vp]),
+    "wisp_cache_ensure_chunks": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp]),
     "wisp_cache_prepare_layer": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
     "wisp_cache_prepare_row": (_i32, [_vp, _vp, _vp, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
     "wisp_cache_prepare_signaled": (_i32, [_vp, _vp, _vp, ctypes.c_uint32, _vp, _i32, _i32, _i64, _i64, _vp, _vp, _vp,

@@ -69,7 +69,7 @@ class ExpertCache:
         # kept as bf16 (cache.py:25-27)
         self.decode_on_load = bool(decode_on_load) and store.bits < 16
         self.cpu_store = cpu_store
-        self.nslots, self.n_static = nslots, n_static
+        self.nslots, self.n_static, self.policy = nslots, n_static, policy
         self.slot_bytes = 3 * store.n * 2 if self.decode_on_load else store.nbytes
         host = store.host
         assert host.dtype == torch.uint8 and host.dim() == 2 and host.is_contiguous() and not host.is_cuda
@@ -218,6 +218,20 @@ class ExpertCache:
         if rc != 0:
             raise RuntimeError(_lib.lib().wisp_last_error().decode())
         return [int(v) for v in slots[: k.size]]
+
+    def ensure_chunks(self, keys, chunk):
+        """ensure(keys[:chunk]), ensure(keys[chunk:2 * chunk]), ... in one call: the slots of all keys, each still
+        holding its key when the call returns (see holds_at_once)."""
+        self.device_end()
+        k = _i64(keys)
+        slots = np.empty(max(k.size, 1), np.int64)
+        _raise(_lib.lib().wisp_cache_ensure_chunks(self._h, _p(k), k.size, chunk, _p(slots), self._stream()))
+        return slots[: k.size].tolist()
+
+    def holds_at_once(self, n):
+        """Whether n different keys, ensured one chunk after another, are all resident at the end: with lru and no more
+        keys than dynamic slots a miss always finds a slot that is older than this sequence."""
+        return self.policy == "lru" and n <= self.nslots - self.n_static
 
     def prepare_layer(self, keys, weights, meta_host: torch.Tensor, meta_dev: torch.Tensor):
         """One layer's host step of the graph decoder (graphdec.py:216-231) in one native call:

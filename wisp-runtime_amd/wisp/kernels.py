@@ -17,6 +17,8 @@ they are accepted and ignored (launch shapes are set by wisp_set_tuning).
 
 from __future__ import annotations
 
+import array
+
 import torch
 
 from . import _lib
@@ -239,9 +241,46 @@ def _prefill_chunks(uniq, first, count, chunk=None):
     return ex[o], start[o], cnt[o]
 
 
+_PLAN_IDS, _PLAN_ABSENT = 512, -(1 << 31)
+_PLAN_SEL = {torch.int64: 8, torch.int32: 4}
+
+
+def _plan_table(expert_slots):
+    """{expert id: slot} as the GPU planner's int32 table (slot of id i), or None where it has no such form:
+    an id outside [0, 512) or a slot that is no int32."""
+    try:
+        hi = max(expert_slots)
+        if min(expert_slots) < 0 or hi >= _PLAN_IDS:
+            return None
+        t = [_PLAN_ABSENT] * (int(hi) + 1)
+        for e, s in expert_slots.items():
+            t[e] = s
+        return array.array("i", t)
+    except (TypeError, OverflowError, ValueError):
+        return None
+
+
+def _prefill_routed(pool, table, x, sel, rw, H, I, bits, group, out, acc, max_pairs):
+    """The launches of a prefill whose routing (sel int64 or int32, rw of a float dtype, both contiguous) is in device
+    memory: the plan, the two GEMMs and the combine."""
+    T, k = sel.shape
+    L = _lib.lib()
+    dev = x.device
+    ws = torch.empty(L.wisp_prefill_routed_ws_bytes(T, k, max_pairs, len(table), H, I), dtype=torch.uint8, device=dev)
+    _lib.check(
+        L.wisp_moe_prefill_routed(
+            _lib.ptr(pool), pool.stride(0), pool.shape[0], _lib.ptr(sel), _PLAN_SEL[sel.dtype], _lib.ptr(rw),
+            _X_DTYPES[rw.dtype], table.buffer_info()[0], len(table), max_pairs, _lib.ptr(x), T, k, H, I, bits, group,
+            _lib.ptr(ws), _lib.ptr(out), _lib.ptr(acc), _lib.stream(dev),
+        ),
+        "moe_prefill",
+    )
+
+
 def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=None):
     """Grouped MoE over T tokens (the dequant + F.linear loop of moe.py:131-151 as three
-    launches). x: [T, H] bf16; sel: [T, k] expert ids; rw: [T, k] routing weights;
+    launches, and a fourth that groups the pairs where `sel` is on the GPU; a routing in host
+    memory is grouped there). x: [T, H] bf16; sel: [T, k] expert ids; rw: [T, k] routing weights;
     expert_slots: {expert id: slot} for the experts to run (others are skipped).
     Returns bf16 [T, H] = per token sum over its experts (ascending id) of
     w * down(SiLU(gate x) * up x); with `acc` (fp32 [T, H]) the sum is added to it instead
@@ -256,6 +295,22 @@ def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=No
         raise TypeError(f"x must be bfloat16 (got {x.dtype})")
     x = x.contiguous()
     T, k = sel.shape
+    # the GPU planner's forms; every other one (ids past its table, odd dtypes and shapes, and what the kernels refuse)
+    # is planned on the host
+    if (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k < 1 << 31 and k <= 32 and x.shape[0] >= T
+            and rw.numel() == T * k and rw.is_floating_point() and expert_slots and group == 128 and H % 256 == 0
+            and I % 128 == 0):
+        table = _plan_table(expert_slots)
+        if table is not None:
+            if acc is None:
+                out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+            else:
+                assert acc.dtype == torch.float32 and acc.shape == (T, H) and acc.is_contiguous()
+                out = None
+            w = rw.detach().reshape(-1).to(dev)
+            w = w.contiguous() if w.dtype in _X_DTYPES else w.to(torch.float32)
+            _prefill_routed(pool, table, x, sel.detach().contiguous(), w, H, I, bits, group, out, acc, T * k)
+            return acc if out is None else out
     sel_cpu = sel.detach().cpu().numpy()
     experts = sorted(int(e) for e in expert_slots)
     order, tok, back, uniq, first, count = _prefill_plan(sel_cpu, experts, k)

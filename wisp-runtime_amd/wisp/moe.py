@@ -184,9 +184,10 @@ class PagedMoEBlock(nn.Module):
 
     def _forward_dequant(self, x, rw, sel, pred, B, T, H):
         """Several tokens (moe.py:82-151, 'transfer' policy), experts paged in chunks of rt.chunk.
-        4/3/2-bit experts with group 128: the grouped prefill kernels (dequant into LDS + bf16
-        MFMA, three launches per chunk, fp32 accumulation across chunks). Otherwise: per routed
-        expert, dequantize its slot and run three bf16 GEMMs on its tokens."""
+        4/3/2-bit experts with group 128: the grouped prefill kernels, once for all experts where
+        the cache keeps them all through the chunks' paging steps, else once per chunk (fp32
+        accumulation across chunks). Otherwise: per routed expert, dequantize its slot and run
+        three bf16 GEMMs on its tokens."""
         rt, cache = self.rt, self.rt.cache
         sel_cpu = sel.cpu()
         self._record(sel_cpu)
@@ -196,6 +197,15 @@ class PagedMoEBlock(nn.Module):
         if st.bits in (2, 3, 4) and st.group == 128 and not cache.decode_on_load and x.dtype == torch.bfloat16:
             from .kernels import moe_prefill
 
+            if cache.holds_at_once(len(keys)):
+                # every routed expert stays resident through the chunks' paging steps: one set of launches for all
+                slots = cache.ensure_chunks(keys, rt.chunk)
+                y = moe_prefill(cache.gpu, {kk - base: s for kk, s in zip(keys, slots)}, x, sel, rw, st.n, H, self.I,
+                                st.bits, st.group)
+                rt.stats["gpu_experts"] += len(keys)
+                if pred is not None:
+                    self._prefetch_next(pred.cpu(), slots[(len(keys) - 1) // rt.chunk * rt.chunk :])
+                return y.view(B, T, H)
             acc = torch.zeros((x.shape[0], H), dtype=torch.float32, device=x.device)
             used = []
             for i in range(0, len(keys), rt.chunk):

@@ -176,3 +176,24 @@ def test_block_runs_all_experts_at_once_where_the_cache_holds_them(nslots, n_sta
         assert err <= 2.0**-8, (step, err)
     for c in caches:
         c.free()
+
+
+# the LDS-DMA GEMMs at every code width: one and several steps, more than 16 K groups, passes of 1 to 8 token tiles and
+# several of them, and an odd number of K groups in the down projection (its register form beside them)
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("E,H,I,T,k", [(3, 256, 256, 2, 1), (4, 512, 512, 90, 2), (3, 4352, 256, 20, 2), (2, 256, 2304, 40, 1),
+                                       (2, 256, 2176, 30, 2), (3, 256, 384, 200, 2), (2, 1024, 256, 300, 2)])
+def test_prefill_dma_every_width(bits, E, H, I, T, k):
+    n = H * I
+    rng = np.random.default_rng(E * H + I + T + bits)
+    pool = np.stack([O.quantize((rng.standard_normal(3 * n) * 0.03).astype(np.float32), bits, 128) for _ in range(E)])
+    sel, rw = O.route(rng.standard_normal((T, E)).astype(np.float32), k)
+    x = O.f32_to_bf16_bits(rng.standard_normal((T, H)).astype(np.float32)).reshape(T, H)
+    ref = O.moe_prefill_f64(pool, {e: e for e in range(E)}, x, sel, rw, H, I, bits)
+    xt = torch.from_numpy(x.view(np.int16)).view(torch.bfloat16).to(DEV)
+    for on in ("cpu", DEV):
+        got = kernels.moe_prefill(torch.from_numpy(pool).to(DEV), {e: e for e in range(E)}, xt,
+                                  torch.from_numpy(sel).to(on), torch.from_numpy(rw).to(DEV), n, H, I, bits)
+        # the oracle's activation is rounded to bf16 as the kernels' is; one more rounding of the result
+        err = np.linalg.norm(got.double().cpu().numpy() - ref) / np.linalg.norm(ref)
+        assert err <= 2.0**-8, (on, err)

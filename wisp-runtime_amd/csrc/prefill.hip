@@ -35,7 +35,7 @@
 // MFMA 16x16x32 bf16 lane layout (lane l): A[row l%16][k 8*(l/16) + 0..7],
 // B[k 8*(l/16) + 0..7][col l%16], D[row 4*(l/16) + 0..3][col l%16].
 // With the weights read once per expert the path is HBM-bound for T <= 512.
-// 4-bit codes with an even number of K groups (the Qwen3 shapes) take the LDS-DMA
+// GEMMs over an even number of K groups (the Qwen3 shapes) take the LDS-DMA
 // form of the two GEMMs (k_pf_gate_up_dmag / k_pf_down_dmag, described at
 // pf_gemm_dmag): the codes of a K step arrive as whole 128-byte lines straight into
 // LDS, one step ahead, and the scales with them.
@@ -75,57 +75,6 @@ struct Prefill {
 __device__ __forceinline__ f32x4_t mfma16(uint4 a, uint4 b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
                                                     c, 0, 0, 0);
-}
-
-// byte N of v as a float (v_cvt_f32_ubyteN: one instruction, no extract)
-__device__ __forceinline__ float ubyte0(uint32_t v) { float r; asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(r) : "v"(v)); return r; }
-__device__ __forceinline__ float ubyte1(uint32_t v) { float r; asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(r) : "v"(v)); return r; }
-__device__ __forceinline__ float ubyte2(uint32_t v) { float r; asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(v)); return r; }
-__device__ __forceinline__ float ubyte3(uint32_t v) { float r; asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(v)); return r; }
-template <int B>
-__device__ __forceinline__ float ubyte(uint32_t v) {
-    return B == 0 ? ubyte0(v) : B == 1 ? ubyte1(v) : B == 2 ? ubyte2(v) : ubyte3(v);
-}
-
-// Dequantize 32 consecutive weights (one chunk) to 16 bf16 pairs, bit-exact with
-// the dequant kernel: w = RTNE_bf16(fp32(q*s) + m). q*s is exact in binary32
-// (q < 16, s an fp16 value), so a fused multiply-add rounds exactly where the
-// separate multiply and add would. 4- and 2-bit codes are first spread one per
-// byte, so that each becomes a float with one v_cvt_f32_ubyteN.
-template <int BITS>
-__device__ __forceinline__ void dequant_chunk(const uint32_t* d, float s, float m, uint32_t* out) {
-    if constexpr (BITS == 4) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t e = d[w] & 0x0F0F0F0Fu;         // codes 8w, 8w+2, 8w+4, 8w+6
-            const uint32_t o = (d[w] >> 4) & 0x0F0F0F0Fu;  // codes 8w+1, 8w+3, 8w+5, 8w+7
-            out[4 * w + 0] = pack_bf16x2(__builtin_fmaf(ubyte<0>(e), s, m), __builtin_fmaf(ubyte<0>(o), s, m));
-            out[4 * w + 1] = pack_bf16x2(__builtin_fmaf(ubyte<1>(e), s, m), __builtin_fmaf(ubyte<1>(o), s, m));
-            out[4 * w + 2] = pack_bf16x2(__builtin_fmaf(ubyte<2>(e), s, m), __builtin_fmaf(ubyte<2>(o), s, m));
-            out[4 * w + 3] = pack_bf16x2(__builtin_fmaf(ubyte<3>(e), s, m), __builtin_fmaf(ubyte<3>(o), s, m));
-        }
-    } else if constexpr (BITS == 2) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            uint32_t f[4];  // f[j] byte b = code 16w + 4b + j
-#pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = (d[w] >> (2 * j)) & 0x03030303u;
-#define WISP_Q2(B)                                                                                      \
-    out[8 * w + 2 * B] = pack_bf16x2(__builtin_fmaf(ubyte<B>(f[0]), s, m), __builtin_fmaf(ubyte<B>(f[1]), s, m));  \
-    out[8 * w + 2 * B + 1] = pack_bf16x2(__builtin_fmaf(ubyte<B>(f[2]), s, m), __builtin_fmaf(ubyte<B>(f[3]), s, m));
-            WISP_Q2(0)
-            WISP_Q2(1)
-            WISP_Q2(2)
-            WISP_Q2(3)
-#undef WISP_Q2
-        }
-    } else {
-        uint32_t q[32];
-        chunk_codes<BITS>(d, q);
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            out[i] = pack_bf16x2(__builtin_fmaf((float)q[2 * i], s, m), __builtin_fmaf((float)q[2 * i + 1], s, m));
-    }
 }
 
 // Group u's (slot, first pair, count). Returns 0 for a group whose pair range is
@@ -200,10 +149,7 @@ __device__ __forceinline__ void pf_stage_scales(const uint16_t* sc, int64_t mn_o
 template <int BITS>
 __device__ __forceinline__ void pf_bfrag(const uint32_t* cd, uint32_t sm, uint4* b) {
     uint32_t v[16];
-    if constexpr (BITS == 3)
-        dequant_chunk<BITS>(cd, h2f((uint16_t)(sm & 0xFFFFu)), h2f((uint16_t)(sm >> 16)), v);
-    else
-        dequant32<BITS>(cd, sm, v);
+    dequant32<BITS>(cd, sm, v);
 #pragma unroll
     for (int s = 0; s < 4; ++s) b[s] = make_uint4(v[4 * s], v[4 * s + 1], v[4 * s + 2], v[4 * s + 3]);
 }
@@ -493,17 +439,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 }
 
 // ===========================================================================
-// LDS-DMA form (4-bit codes, an even number nk <= kPfSmSteps of K groups):
+// LDS-DMA form (an even number nk of K groups):
 // pf_gemm_dmag, k_pf_gate_up_dmag, k_pf_down_dmag.
 // A workgroup of 4 waves owns 128 weight rows, a wave 32 (two 16-row tiles).
 // A K step is one pair of groups (256 K): for each row the step's codes are one
-// whole 128-byte line, and every line is fetched by ONE request:
+// whole 128-byte line at 4 bits (96 and 64 bytes at 3 and 2), and every line is fetched by ONE request:
 // global_load_lds_dwordx4 moves 64 lanes x 16 bytes = 8 rows x 128 bytes
 // straight into LDS (no VGPRs held while in flight), where each lane then reads
 // its MFMA fragment chunk. (Loads into registers in the fragment layout can only
 // cover 16 rows x 64 bytes per instruction, i.e. every line in two halves, which
 // measured 23 % slower in a loads-only run.)
-//   * codes: per wave one private slot of 4 KB codes + 256 B of the rows' fp16
+//   * codes: per wave one private slot (4 KB at 4 bits) + 256 B of the rows' fp16
 //     scale and min pairs; it is read into registers at the step's start and
 //     then refilled with the next step's codes, which have the whole step to
 //     arrive.
@@ -570,12 +516,68 @@ struct PfDma {
     const uint8_t* cb[2];  // code base of row tile jj (its first row, pair 0), wave-uniform
     const uint8_t* sb;     // scale base: fp16 scales of the wave's row 0, pair 0, wave-uniform
     int64_t rowb;          // code bytes of one row
-    uint32_t voc;          // lane code offset: row lane>>3 of an 8-row block, piece (lane&7)^(lane>>3)
+    uint32_t voc[3];       // lane code offsets (pf_issue_codes)
     uint32_t vos;          // lane scale offset: lanes 0-31 scale pair, 32-63 min pair of the wave's row lane&31
 };
 
-// per wave: one slot of 4 KB codes + 256 B scales
-constexpr int kDmaSlot = 4096 + 256;
+// Per wave: one slot of the step's codes (32 rows of 64 * BITS / 2 bytes) and 256 B of scales and mins.
+template <int BITS>
+constexpr int kDmaSlot = 32 * 32 * BITS + 256;
+
+// A row's codes of a step (two quant groups) are 2 * BITS pieces of 16 bytes, and BITS DMA instructions fetch the
+// wave's 32 rows. 4 bits: 8 rows x 8 pieces per instruction, piece p of row r stored at position p ^ (r & 7).
+// 2 bits: 16 rows x 4 pieces, p at p ^ (r/2 & 3) (two rows fill the 32 banks). 3 bits: the 192 pieces in row order,
+// unswizzled (a row is 24 banks; a fragment is 12 bytes); a row's pieces straddle instructions, so each has its own
+// lane offsets, the second tile's base included.
+template <int BITS>
+__device__ __forceinline__ void pf_code_offsets(PfDma& R, int lane) {
+    if constexpr (BITS == 4) {
+        R.voc[0] = (uint32_t)((lane >> 3) * R.rowb + 16 * ((lane & 7) ^ (lane >> 3)));
+    } else if constexpr (BITS == 2) {
+        R.voc[0] = (uint32_t)((lane >> 2) * R.rowb + 16 * ((lane & 3) ^ ((lane >> 3) & 3)));
+    } else {
+        const uint32_t second = (uint32_t)(R.cb[1] - R.cb[0]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int idx = 64 * i + lane, row = idx / 6, p = idx - 6 * row;
+            R.voc[i] = (uint32_t)((row & 15) * R.rowb + 16 * p) + (row >= 16 ? second : 0u);
+        }
+    }
+}
+template <int BITS>
+__device__ __forceinline__ void pf_issue_codes(const PfDma& R, uint32_t ring_l, int st) {
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) {
+        const uint8_t* b = BITS == 4 ? R.cb[i >> 1] + (i & 1) * 8 * R.rowb : BITS == 2 ? R.cb[i] : R.cb[0];
+        dma16s(ring_l + i * 1024, b + (int64_t)st * (32 * BITS), R.voc[BITS == 3 ? i : 0]);
+    }
+    dma4s(ring_l + 1024 * BITS, R.sb + st * 4, R.vos);
+}
+// the lane's chunks (row n of tile jj, chunk g of both groups) and packed scales from the wave's slot
+template <int BITS>
+__device__ __forceinline__ void pf_read_slot(const uint8_t* ring, int n, int g, uint32_t (*cd)[2][BITS], uint32_t (*sm)[2]) {
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+        const uint8_t* row = ring + (16 * jj + n) * (32 * BITS);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (BITS == 4) {
+                const uint4 v = *reinterpret_cast<const uint4*>(row + 16 * ((4 * h + g) ^ (n & 7)));
+                cd[jj][h][0] = v.x; cd[jj][h][1] = v.y; cd[jj][h][2] = v.z; cd[jj][h][3] = v.w;
+            } else if constexpr (BITS == 2) {
+                const uint2 v = *reinterpret_cast<const uint2*>(row + 16 * ((2 * h + (g >> 1)) ^ ((n >> 1) & 3)) + 8 * (g & 1));
+                cd[jj][h][0] = v.x; cd[jj][h][1] = v.y;
+            } else {
+                const uint32_t* v = reinterpret_cast<const uint32_t*>(row + 48 * h + 12 * g);
+                cd[jj][h][0] = v[0]; cd[jj][h][1] = v[1]; cd[jj][h][2] = v[2];
+            }
+        }
+        const uint32_t sp = *reinterpret_cast<const uint32_t*>(ring + 1024 * BITS + 4 * (16 * jj + n));
+        const uint32_t mp = *reinterpret_cast<const uint32_t*>(ring + 1024 * BITS + 128 + 4 * (16 * jj + n));
+        sm[jj][0] = __builtin_amdgcn_perm(mp, sp, 0x05040100u);
+        sm[jj][1] = __builtin_amdgcn_perm(mp, sp, 0x07060302u);
+    }
+}
 
 // NT token tiles, NW waves of two 16-row tiles each; abase: uniform A base (group 0),
 // avo[k]: the lane's A offset for its k-th piece; abuf: 2 x NT*16 rows x 256 B;
@@ -583,49 +585,33 @@ constexpr int kDmaSlot = 4096 + 256;
 // A(G) = the RPTG token DMAs of group G):
 //   wait all, barrier | A(2st+1) | read the slot | C(st+1) | group 2st
 //   wait A(2st+1) (C(st+1) stays in flight), barrier | A(2st+2) | group 2st+1
-template <int NT, int NW>
+template <int BITS, int NT, int NW>
 __device__ __forceinline__ void pf_gemm_dmag(const PfDma& R, const uint8_t* abase, const uint32_t* avo, uint8_t* abuf,
                                              uint8_t* ring, int nk, f32x4_t (*acc)[2]) {
     constexpr int RPTG = 4 * NT / NW;  // A DMA instructions per wave and group
     static_assert(RPTG >= 1 && (4 * NT) % NW == 0, "A pieces per wave");
     constexpr int ABUF = NT * 16 * 256;
-    constexpr int CN = 5;  // code and scale DMA instructions per step
+    constexpr int CN = BITS + 1;  // code and scale DMA instructions per step
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nsteps = nk >> 1;
 #pragma unroll
     for (int mt = 0; mt < NT; ++mt) acc[mt][0] = acc[mt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint32_t ring_l = lds_addr(ring), abuf_l = lds_addr(abuf);
-    auto issue_c = [&](int st) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            dma16s(ring_l + i * 1024, R.cb[i >> 1] + (i & 1) * 8 * R.rowb + (int64_t)st * 128, R.voc);
-        dma4s(ring_l + 4096, R.sb + st * 4, R.vos);
-    };
+    auto issue_c = [&](int st) { pf_issue_codes<BITS>(R, ring_l, st); };
     auto issue_a = [&](int G) {
         const uint32_t dst = abuf_l + (G & 1) * ABUF;
 #pragma unroll
         for (int k = 0; k < RPTG; ++k) dma16s(dst + 1024 * (wv + NW * k), abase + G * 256, avo[k]);
     };
-    const uint32_t co0 = 128 * n + 16 * ((0 + g) ^ (n & 7)), co1 = 128 * n + 16 * ((4 + g) ^ (n & 7));
     issue_c(0);
     issue_a(0);
     for (int st = 0; st < nsteps; ++st) {
         wait_vm<0>();     // C(st) and A(2st)
         __syncthreads();  // every wave's part of A(2st) landed; every read of group 2st-1 ended
         issue_a(2 * st + 1);
-        uint32_t cd[2][2][4], sm[2][2];
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            const uint4 v0 = *reinterpret_cast<const uint4*>(ring + 2048 * jj + co0);
-            const uint4 v1 = *reinterpret_cast<const uint4*>(ring + 2048 * jj + co1);
-            cd[jj][0][0] = v0.x; cd[jj][0][1] = v0.y; cd[jj][0][2] = v0.z; cd[jj][0][3] = v0.w;
-            cd[jj][1][0] = v1.x; cd[jj][1][1] = v1.y; cd[jj][1][2] = v1.z; cd[jj][1][3] = v1.w;
-            const uint32_t sp = *reinterpret_cast<const uint32_t*>(ring + 4096 + 4 * (16 * jj + n));
-            const uint32_t mp = *reinterpret_cast<const uint32_t*>(ring + 4096 + 128 + 4 * (16 * jj + n));
-            sm[jj][0] = __builtin_amdgcn_perm(mp, sp, 0x05040100u);
-            sm[jj][1] = __builtin_amdgcn_perm(mp, sp, 0x07060302u);
-        }
+        uint32_t cd[2][2][BITS], sm[2][2];
+        pf_read_slot<BITS>(ring, n, g, cd, sm);
         wait_lgkm0();  // the slot is read: it may be refilled
         if (st + 1 < nsteps) issue_c(st + 1);
 #pragma unroll
@@ -646,7 +632,7 @@ __device__ __forceinline__ void pf_gemm_dmag(const PfDma& R, const uint8_t* abas
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj) {
                 uint4 b[4];
-                pf_bfrag<4>(cd[jj][h], sm[jj][h], b);
+                pf_bfrag<BITS>(cd[jj][h], sm[jj][h], b);
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -670,36 +656,30 @@ __device__ __forceinline__ void pf_gemm_dmag(const PfDma& R, const uint8_t* abas
 //   wait all, barrier | A(4st+4) | stage 4st+3
 // avo[k]: the lane's offset of its k-th A piece for group 0, half 0 (the lane's logical
 // piece p = 2g + s' maps to the group's byte 16 * (4g + 2hh + s')).
-template <int NT, int NW>
+template <int BITS, int NT, int NW>
 __device__ __forceinline__ void pf_gemm_dmag_h(const PfDma& R, const uint8_t* abase, const uint32_t* avo,
                                                uint8_t* abuf, uint8_t* ring, int nk, f32x4_t (*acc)[2]) {
     constexpr int RPTS = 2 * NT / NW;  // A DMA instructions per wave and stage
     static_assert(RPTS >= 1 && (2 * NT) % NW == 0, "A pieces per wave");
     constexpr int SBUF = NT * 16 * 128;
-    constexpr int CN = 5;
+    constexpr int CN = BITS + 1;
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nsteps = nk >> 1, nst = 2 * nk;
 #pragma unroll
     for (int mt = 0; mt < NT; ++mt) acc[mt][0] = acc[mt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint32_t ring_l = lds_addr(ring), abuf_l = lds_addr(abuf);
-    auto issue_c = [&](int st) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            dma16s(ring_l + i * 1024, R.cb[i >> 1] + (i & 1) * 8 * R.rowb + (int64_t)st * 128, R.voc);
-        dma4s(ring_l + 4096, R.sb + st * 4, R.vos);
-    };
+    auto issue_c = [&](int st) { pf_issue_codes<BITS>(R, ring_l, st); };
     auto issue_a = [&](int q) {
         const uint32_t dst = abuf_l + (q & 1) * SBUF;
         const uint8_t* src = abase + (q >> 1) * 256 + (q & 1) * 32;
 #pragma unroll
         for (int k = 0; k < RPTS; ++k) dma16s(dst + 1024 * (wv + NW * k), src, avo[k]);
     };
-    const uint32_t co0 = 128 * n + 16 * ((0 + g) ^ (n & 7)), co1 = 128 * n + 16 * ((4 + g) ^ (n & 7));
     issue_c(0);
     issue_a(0);
     for (int st = 0; st < nsteps; ++st) {
-        uint32_t cd[2][2][4], sm[2][2];
+        uint32_t cd[2][2][BITS], sm[2][2];
         uint4 b[2][4];  // B fragments of the current group, kept across its half-group barrier
 #pragma unroll
         for (int hq = 0; hq < 4; ++hq) {
@@ -708,24 +688,14 @@ __device__ __forceinline__ void pf_gemm_dmag_h(const PfDma& R, const uint8_t* ab
             __syncthreads();  // every wave's part of A(q) landed; every read of stage q-1 ended
             if (q + 1 < nst) issue_a(q + 1);
             if (hq == 0) {
-#pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
-                    const uint4 v0 = *reinterpret_cast<const uint4*>(ring + 2048 * jj + co0);
-                    const uint4 v1 = *reinterpret_cast<const uint4*>(ring + 2048 * jj + co1);
-                    cd[jj][0][0] = v0.x; cd[jj][0][1] = v0.y; cd[jj][0][2] = v0.z; cd[jj][0][3] = v0.w;
-                    cd[jj][1][0] = v1.x; cd[jj][1][1] = v1.y; cd[jj][1][2] = v1.z; cd[jj][1][3] = v1.w;
-                    const uint32_t sp = *reinterpret_cast<const uint32_t*>(ring + 4096 + 4 * (16 * jj + n));
-                    const uint32_t mp = *reinterpret_cast<const uint32_t*>(ring + 4096 + 128 + 4 * (16 * jj + n));
-                    sm[jj][0] = __builtin_amdgcn_perm(mp, sp, 0x05040100u);
-                    sm[jj][1] = __builtin_amdgcn_perm(mp, sp, 0x07060302u);
-                }
+                pf_read_slot<BITS>(ring, n, g, cd, sm);
                 wait_lgkm0();  // the slot is read: it may be refilled
                 if (st + 1 < nsteps) issue_c(st + 1);
             }
             const uint8_t* A = abuf + (q & 1) * SBUF;
             if (hh == 0) {
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj) pf_bfrag<4>(cd[jj][h], sm[jj][h], b[jj]);
+                for (int jj = 0; jj < 2; ++jj) pf_bfrag<BITS>(cd[jj][h], sm[jj][h], b[jj]);
             }
 #pragma unroll
             for (int mt = 0; mt < NT; ++mt) {
@@ -742,7 +712,7 @@ __device__ __forceinline__ void pf_gemm_dmag_h(const PfDma& R, const uint8_t* ab
     }
 }
 
-template <int MT, int NW, bool GATE_UP, class Epi>
+template <int BITS, int MT, int NW, bool GATE_UP, class Epi>
 __device__ __forceinline__ void pf_dmag_passes(const Prefill& F, const PfDma& R, int p0, int cnt, uint8_t* ab,
                                                uint8_t* ringw, int nk, int bz, int nz, Epi epi) {
     const int lane = threadIdx.x & 63;
@@ -773,7 +743,7 @@ __device__ __forceinline__ void pf_dmag_passes(const Prefill& F, const PfDma& R,
                 }
             }
             f32x4_t acc[NT][2];
-            pf_gemm_dmag<NT, NW>(R, abase, avo, ab, ringw, nk, acc);
+            pf_gemm_dmag<BITS, NT, NW>(R, abase, avo, ab, ringw, nk, acc);
             epi(acc, mb);
         };
         // 5..8 tiles: staged half a group at a time (pf_gemm_dmag_h); lane l of A DMA
@@ -799,7 +769,7 @@ __device__ __forceinline__ void pf_dmag_passes(const Prefill& F, const PfDma& R,
             if constexpr (GATE_UP) abase = uniform_ptr(F.x);
             else abase = uniform_ptr(F.act + (int64_t)p0 * F.I);
             f32x4_t acc[NT][2];
-            pf_gemm_dmag_h<NT, NW>(R, abase, avo, ab, ringw, nk, acc);
+            pf_gemm_dmag_h<BITS, NT, NW>(R, abase, avo, ab, ringw, nk, acc);
             epi(acc, mb);
         };
         bool half = false;
@@ -817,11 +787,11 @@ __device__ __forceinline__ void pf_dmag_passes(const Prefill& F, const PfDma& R,
     }
 }
 
-template <int MT, int NW>
+template <int BITS, int MT, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_gate_up_dmag(const Prefill F) {
     constexpr int RWG = 32 * NW, HR = RWG / 2, CW = 16;
     __shared__ uint4 abuf[2 * (MT > 4 ? 4 : MT) * 16 * 16];  // 5..8 tiles: staged per half group
-    __shared__ uint4 ring[NW * kDmaSlot / 16];
+    __shared__ uint4 ring[NW * kDmaSlot<BITS> / 16];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
     // one-dimensional launch of (I / HR) x gy x gz workgroups: an item's row blocks share an
@@ -840,17 +810,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const uint8_t* base = F.pool + (int64_t)slot * F.slot_bytes;
     const int nk = F.H / 128;
     PfDma R;
-    R.rowb = (int64_t)F.H / 2;
+    R.rowb = (int64_t)F.H * BITS / 8;
     R.cb[0] = uniform_ptr(base + (int64_t)c0 * R.rowb);
     R.cb[1] = uniform_ptr(base + F.nmb + (int64_t)c0 * R.rowb);
-    R.voc = (uint32_t)((lane >> 3) * R.rowb + 16 * ((lane & 7) ^ (lane >> 3)));
+    pf_code_offsets<BITS>(R, lane);
     const uint8_t* sc = base + 3 * F.nmb;
     R.sb = uniform_ptr(sc + (int64_t)c0 * nk * 2);
     R.vos = (uint32_t)((lane >= 32 ? 3 * (int64_t)F.NGM * 2 : 0) + ((lane & 31) >> 4) * (int64_t)F.NGM * 2 +
                        (lane & 15) * nk * 2);
-    uint8_t* ringw = reinterpret_cast<uint8_t*>(ring) + wv * kDmaSlot;
+    uint8_t* ringw = reinterpret_cast<uint8_t*>(ring) + wv * kDmaSlot<BITS>;
     uint8_t* ab = reinterpret_cast<uint8_t*>(abuf);
-    pf_dmag_passes<MT, NW, true>(F, R, p0, cnt, ab, ringw, nk, bz, F.gz, [&](auto& acc, int mb) {
+    pf_dmag_passes<BITS, MT, NW, true>(F, R, p0, cnt, ab, ringw, nk, bz, F.gz, [&](auto& acc, int mb) {
         constexpr int NT = sizeof(acc) / sizeof(acc[0]);
 #pragma unroll
         for (int mt = 0; mt < NT; ++mt)
@@ -862,11 +832,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     });
 }
 
-template <int MT, int NW>
+template <int BITS, int MT, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_down_dmag(const Prefill F) {
     constexpr int RWG = 32 * NW, RW = 32;
     __shared__ uint4 abuf[2 * (MT > 4 ? 4 : MT) * 16 * 16];  // 5..8 tiles: staged per half group
-    __shared__ uint4 ring[NW * kDmaSlot / 16];
+    __shared__ uint4 ring[NW * kDmaSlot<BITS> / 16];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
     // one-dimensional launch of (H / RWG) x gy x gz workgroups: an item's row blocks share an
@@ -885,16 +855,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const uint8_t* base = F.pool + (int64_t)slot * F.slot_bytes;
     const int nk = F.I / 128;
     PfDma R;
-    R.rowb = (int64_t)F.I / 2;
+    R.rowb = (int64_t)F.I * BITS / 8;
     R.cb[0] = uniform_ptr(base + 2 * F.nmb + (int64_t)h0 * R.rowb);
     R.cb[1] = uniform_ptr(base + 2 * F.nmb + (int64_t)(h0 + 16) * R.rowb);
-    R.voc = (uint32_t)((lane >> 3) * R.rowb + 16 * ((lane & 7) ^ (lane >> 3)));
+    pf_code_offsets<BITS>(R, lane);
     const uint8_t* sc = base + 3 * F.nmb;
     R.sb = uniform_ptr(sc + (2 * (int64_t)F.NGM + (int64_t)h0 * nk) * 2);
     R.vos = (uint32_t)((lane >= 32 ? 3 * (int64_t)F.NGM * 2 : 0) + (lane & 31) * nk * 2);
-    uint8_t* ringw = reinterpret_cast<uint8_t*>(ring) + wv * kDmaSlot;
+    uint8_t* ringw = reinterpret_cast<uint8_t*>(ring) + wv * kDmaSlot<BITS>;
     uint8_t* ab = reinterpret_cast<uint8_t*>(abuf);
-    pf_dmag_passes<MT, NW, false>(F, R, p0, cnt, ab, ringw, nk, bz, F.gz, [&](auto& acc, int mb) {
+    pf_dmag_passes<BITS, MT, NW, false>(F, R, p0, cnt, ab, ringw, nk, bz, F.gz, [&](auto& acc, int mb) {
         constexpr int NT = sizeof(acc) / sizeof(acc[0]);
 #pragma unroll
         for (int mt = 0; mt < NT; ++mt)
@@ -1122,41 +1092,34 @@ __global__ __launch_bounds__(64 * kPlanWaves) void k_pf_plan(const ST* __restric
 // share a larger group's passes
 template <int BITS, int MT>
 static void launch_pf_mt(const Prefill& F, int ngroups, int max_group, hipStream_t st) {
-    if constexpr (BITS == 4) {
-        const unsigned z = (unsigned)std::min(64, std::max(1, (max_group + MT * 16 - 1) / (MT * 16)));
-        // the LDS-DMA form: an even number of K groups in both GEMMs, at most kPfSmSteps, and
-        // x and act addressable with 32-bit offsets
-        const int nkg = F.H / 128, nkd = F.I / 128;
-        const bool off32 = (int64_t)F.T * F.H * 2 < (int64_t(1) << 31) && (int64_t)F.P * F.I * 2 < (int64_t(1) << 31);
-        if (nkg % 2 == 0 && nkd % 2 == 0 && nkg <= kPfSmSteps && nkd <= kPfSmSteps && off32) {
-            // 4-wave workgroups of 128 rows, token tiles staged per quant group: two or three
-            // workgroups share a CU (measured on C5 against 8-wave workgroups with the tile
-            // staged per group pair, one per CU: T = 256 119.7 -> 114.3 us, 512 150.5 -> 142.3)
-            if (F.I % 64 == 0 && F.H % 128 == 0) {
-                Prefill G = F;
-                G.gy = ngroups;
-                G.gz = (int)z;
-                hipLaunchKernelGGL((k_pf_gate_up_dmag<MT, 4>), dim3((unsigned)(F.I / 64) * (unsigned)ngroups * z),
-                                   dim3(256), 0, st, G);
-                hipLaunchKernelGGL((k_pf_down_dmag<MT, 4>), dim3((unsigned)(F.H / 128) * (unsigned)ngroups * z),
-                                   dim3(256), 0, st, G);
-                return;
-            }
-        }
-    }
-    if constexpr (MT > 4) {
-        launch_pf_mt<BITS, 4>(F, ngroups, max_group, st);  // passes of more than 4 tiles: LDS-DMA form only
-        return;
-    }
-    constexpr int MTR = MT > 4 ? 4 : MT;  // the register form's tile count (MT <= 4 here)
+    // The LDS-DMA form takes an even number of K groups (a step is two, and a scale pair one aligned word) and x and
+    // act addressable with 32-bit offsets: every gate_up (H is a multiple of 256) and the down of an even I / 128.
+    // 4-wave workgroups of 128 rows, token tiles staged per quant group: two or three workgroups share a CU (measured
+    // on C5 against 8-wave workgroups with the tile staged per group pair, one per CU: T = 256 119.7 -> 114.3 us, 512
+    // 150.5 -> 142.3). Against the register form, one call
+    // with its plan and combine: 1,000 tokens over 64 experts of 4096 x 1536 at 4 bits (more than 16 K groups) 468 -> 274 us;
+    // 2,000 tokens over 128 of 2048 x 768 449 -> 267 at 3 bits, 512 136 -> 104 at 2, 64 107 -> 92 at 3.
+    const unsigned z = (unsigned)std::min(64, std::max(1, (max_group + MT * 16 - 1) / (MT * 16)));
+    const bool off32 = (int64_t)F.T * F.H * 2 < (int64_t(1) << 31) && (int64_t)F.P * F.I * 2 < (int64_t(1) << 31);
+    Prefill G = F;
+    G.gy = ngroups;
+    G.gz = (int)z;
+    // the register form: passes of at most 4 tiles, 256 rows per workgroup
+    constexpr int MTR = MT > 4 ? 4 : MT;
     constexpr int NW = MTR >= 4 ? 8 : 4, RWG = 256;
-    const unsigned z = (unsigned)std::min(64, std::max(1, (max_group + MTR * 16 - 1) / (MTR * 16)));
-    const dim3 ggu((unsigned)(F.I / (RWG / 2)), (unsigned)ngroups, z), gdn((unsigned)(F.H / RWG), (unsigned)ngroups, z);
-    if (F.H / 128 <= kPfSmSteps)
+    const unsigned zr = (unsigned)std::min(64, std::max(1, (max_group + MTR * 16 - 1) / (MTR * 16)));
+    const dim3 ggu((unsigned)(F.I / (RWG / 2)), (unsigned)ngroups, zr), gdn((unsigned)(F.H / RWG), (unsigned)ngroups, zr);
+    if (off32)
+        hipLaunchKernelGGL((k_pf_gate_up_dmag<BITS, MT, 4>), dim3((unsigned)(F.I / 64) * (unsigned)ngroups * z),
+                           dim3(256), 0, st, G);
+    else if (F.H / 128 <= kPfSmSteps)
         hipLaunchKernelGGL((k_pf_gate_up<BITS, MTR, NW, RWG, true>), ggu, dim3(64 * NW), 0, st, F);
     else
         hipLaunchKernelGGL((k_pf_gate_up<BITS, MTR, NW, RWG, false>), ggu, dim3(64 * NW), 0, st, F);
-    if (F.I / 128 <= kPfSmSteps)
+    if (off32 && F.I / 128 % 2 == 0)
+        hipLaunchKernelGGL((k_pf_down_dmag<BITS, MT, 4>), dim3((unsigned)(F.H / 128) * (unsigned)ngroups * z),
+                           dim3(256), 0, st, G);
+    else if (F.I / 128 <= kPfSmSteps)
         hipLaunchKernelGGL((k_pf_down<BITS, MTR, NW, RWG, true>), gdn, dim3(64 * NW), 0, st, F);
     else
         hipLaunchKernelGGL((k_pf_down<BITS, MTR, NW, RWG, false>), gdn, dim3(64 * NW), 0, st, F);

@@ -275,7 +275,32 @@ __device__ __forceinline__ float half_hi_f(uint32_t x) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(x >> 16));
 }
 
-// Dequantize one chunk of 32 codes (BITS = 4 or 2; BITS dwords d, element i at
+// 3-bit: the 24-bit windows of a chunk, masked without the bias: window P holds code PairMap<3>::lo(P) in the low half
+// and code PairMap<3>::hi(P) in the high half at the offsets below (0, 1 or 2; fp16 subnormals need p + 3 <= 10)
+__device__ __forceinline__ void masked_windows3(const uint32_t* d, uint32_t* w) {
+    constexpr uint32_t MA = 0x0007000Eu, MC = 0x001C0007u;  // (c, c+5): p = 1 / 0; (c, c+6): p = 0 / 2
+    const uint32_t d0 = d[0], d1 = d[1], d2 = d[2];
+    const uint32_t v[16] = {(d0 << 1) & MA,
+                            alignbit(d1, d0, 2) & MA,
+                            alignbit(d1, d0, 5) & MA,
+                            alignbit(d1, d0, 8) & MA,
+                            alignbit(d1, d0, 11) & MA,
+                            alignbit(d1, d0, 29) & MA,
+                            d1 & MA,
+                            alignbit(d2, d1, 3) & MA,
+                            alignbit(d2, d1, 6) & MA,
+                            alignbit(d2, d1, 9) & MA,
+                            alignbit(d2, d1, 28) & MC,
+                            alignbit(d2, d1, 31) & MC,
+                            (d2 >> 2) & MC,
+                            (d2 >> 5) & MC,
+                            (d2 >> 8) & MC,
+                            (d2 >> 11) & MC};
+#pragma unroll
+    for (int P = 0; P < 16; ++P) w[P] = v[P];
+}
+
+// Dequantize one chunk of 32 codes (BITS = 4, 3 or 2; BITS dwords d, element i at
 // bit BITS*i) of a group whose fp16 scale s and min m are packed in
 // sm = s | m << 16, into 32 binary32 values in element order: q*s + m rounded
 // once, the value quant.py:76-87 computes (q*s is exact in binary32) before its
@@ -303,8 +328,18 @@ __device__ __forceinline__ void dequant32_f32(const uint32_t* d, uint32_t sm, fl
             v[8 * w + 6] = __builtin_fmaf(half_hi_f(c), s0, m);
             v[8 * w + 7] = __builtin_fmaf(half_hi_f(e), s4, m);
         }
+    } else if constexpr (BITS == 3) {
+        // the windows of chunk_dot_f32<3>: low code at p = 1 (high at 0) for the (c, c + 5) pairs, 0 (2) for (c, c + 6)
+        uint32_t w[16];
+        masked_windows3(d, w);
+        const float s0 = s * 0x1p24f, s1 = s * 0x1p23f, s2 = s * 0x1p22f;
+#pragma unroll
+        for (int P = 0; P < 16; ++P) {
+            v[PairMap<3>::lo(P)] = __builtin_fmaf(half_lo_f(w[P]), P < 10 ? s1 : s0, m);
+            v[PairMap<3>::hi(P)] = __builtin_fmaf(half_hi_f(w[P]), P < 10 ? s0 : s2, m);
+        }
     } else {
-        static_assert(BITS == 2, "dequant32_f32: 4 or 2 bits");
+        static_assert(BITS == 2, "dequant32_f32: 4, 3 or 2 bits");
         const float sk[4] = {s * 0x1p24f, s * 0x1p22f, s * 0x1p20f, s * 0x1p18f};
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
@@ -376,26 +411,8 @@ __device__ __forceinline__ float chunk_dot_f32<2>(const uint32_t* d, const float
 
 template <>
 __device__ __forceinline__ float chunk_dot_f32<3>(const uint32_t* d, const float* a) {
-    // 24-bit windows, masked without the bias: window P holds code PairMap<3>::lo(P) in the low half and code
-    // PairMap<3>::hi(P) in the high half at the offsets below (0, 1 or 2; fp16 subnormals need p + 3 <= 10)
-    constexpr uint32_t MA = 0x0007000Eu, MC = 0x001C0007u;  // (c, c+5): p = 1 / 0; (c, c+6): p = 0 / 2
-    const uint32_t d0 = d[0], d1 = d[1], d2 = d[2];
-    const uint32_t w[16] = {(d0 << 1) & MA,
-                            alignbit(d1, d0, 2) & MA,
-                            alignbit(d1, d0, 5) & MA,
-                            alignbit(d1, d0, 8) & MA,
-                            alignbit(d1, d0, 11) & MA,
-                            alignbit(d1, d0, 29) & MA,
-                            d1 & MA,
-                            alignbit(d2, d1, 3) & MA,
-                            alignbit(d2, d1, 6) & MA,
-                            alignbit(d2, d1, 9) & MA,
-                            alignbit(d2, d1, 28) & MC,
-                            alignbit(d2, d1, 31) & MC,
-                            (d2 >> 2) & MC,
-                            (d2 >> 5) & MC,
-                            (d2 >> 8) & MC,
-                            (d2 >> 11) & MC};
+    uint32_t w[16];
+    masked_windows3(d, w);
     float s[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};  // by offset p, two chains each
 #pragma unroll
     for (int P = 0; P < 16; ++P) {

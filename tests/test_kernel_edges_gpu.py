@@ -116,6 +116,25 @@ def test_prefill_plan_on_the_gpu_equals_the_hosts(E, k, T, bits, mode):
     assert torch.equal(acc.view(torch.int32), ref.view(torch.int32))
 
 
+def test_prefill_is_planned_on_the_host_where_the_workspace_does_not_fit(monkeypatch):
+    """The GPU plan's workspace has room for all T * k pairs: a call that runs few of them must not need it."""
+    E, k, T, H, I, bits, n = 8, 2, 70, 256, 128, 4, 256 * 128
+    rng = np.random.default_rng(6)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(E)])).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(10)
+    x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
+    sel, rw = _routing(gen, T, E, k)
+    for slots in ({1: 1, 6: 6}, {1: -(1 << 31), 6: 6}):  # and a slot that is the table's mark of an absent expert
+        want = kernels.moe_prefill(pool, slots, x, sel.cpu(), rw, n, H, I, bits)
+        assert torch.equal(kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits).view(torch.int16),
+                           want.view(torch.int16))
+        with monkeypatch.context() as m:
+            m.setattr(kernels, "_plan_workspace", lambda nbytes, dev: None)
+            got = kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_prefill_under_graph_capture_follows_the_routing():
     E, k, T, H, I, bits, n = 8, 2, 70, 256, 128, 4, 256 * 128
     rng = np.random.default_rng(5)

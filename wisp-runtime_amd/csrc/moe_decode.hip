@@ -175,6 +175,22 @@ __device__ __forceinline__ float chunk_dot(const uint32_t* codes, const uint32_t
     return a0 + a1;
 }
 
+// A chunk's share of a row, s * dot + m * sum, with its rounding spelled out so that every kernel that may take a shape gives
+// the same bits: FUSE_S rounds m * sum and fuses the scale's product, else the other way round.
+template <bool FUSE_S>
+__device__ __forceinline__ float chunk_value(float s, float dot, float m, float sum) {
+    return FUSE_S ? __builtin_fmaf(s, dot, __fmul_rn(m, sum)) : __builtin_fmaf(m, sum, __fmul_rn(s, dot));
+}
+// k_gate_up_generic's and k_gate_up_wide's up rows; their gate rows take <false>
+template <int BITS, int XT>
+constexpr bool kFuseUp = XT == WISP_DT_F32 || (XT == WISP_DT_BF16 && BITS != 2);
+
+// a + b, never fused with a product that formed one of them
+__device__ __forceinline__ float add_rn(float a, float b) {
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 // Sum the SPR partials of row-set q (LDS floats src[0..SPR)) across the LPS
 // lanes of its lane group (LPS a power of two <= 16, groups aligned inside a
 // 16-lane DPP row); every lane of the group gets the total. The cross-lane
@@ -197,7 +213,7 @@ __device__ __forceinline__ float group_sum(const float* src, int SPR, int sub, i
 }
 
 // lanes per row-set sum for NQ sums over 64 lanes: a power of two, at most 16
-__device__ __forceinline__ int lanes_per_sum(int NQ) {
+__host__ __device__ __forceinline__ int lanes_per_sum(int NQ) {
     int LPS = 1;
     while (LPS < 16 && LPS * 2 * NQ <= 64) LPS <<= 1;
     return LPS;
@@ -408,7 +424,7 @@ __global__ __launch_bounds__(64 * NW) void k_gate_up_c2(const float* __restrict_
 
 // Kernel 1 for rows of more than 64 chunks (H > 2048, G = 128 * 2^i): one wave = T rows (gate and up) of one
 // expert, CPL = ceil(H / 2048) chunks of a row per lane (chunks lane, lane + 64, ...), every load issued before any use.
-// The arithmetic per chunk is k_gate_up_generic's (fp32 x, exact products); T = 2 where a
+// The arithmetic per chunk and the order of the sums are k_gate_up_generic's (fp32 x, exact products): the same bits. T = 2 where a
 // chunk's 32 x values, unpacked once, and their sum serve two gate and two up rows (at CPL = 4 the registers allow one row).
 // Bound by the codes' bytes and, next, VALU issue: 53.5 MB at H 4096, I 1536, k = 8, 4 bits took 17.1 us with one row per
 // single-wave workgroup and a load loop (k_gate_up_generic), 12.8 here (T = 1: 14.7, T = 4: 14.5), where a plain read of
@@ -460,15 +476,16 @@ __global__ __launch_bounds__(256) void k_gate_up_wide(const float* __restrict__ 
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const float dg = chunk_dot_f32<BITS>(cg[t][c], xf), du = chunk_dot_f32<BITS>(cu[t][c], xf);
-            const float vg = h2f((uint16_t)quad_bcast<0>(sv[t][c])) * dg + h2f((uint16_t)quad_bcast<1>(sv[t][c])) * xs;
-            const float vu = h2f((uint16_t)quad_bcast<2>(sv[t][c])) * du + h2f((uint16_t)quad_bcast<3>(sv[t][c])) * xs;
+            const float vg = chunk_value<false>(h2f((uint16_t)quad_bcast<0>(sv[t][c])), dg, h2f((uint16_t)quad_bcast<1>(sv[t][c])), xs);
+            const float vu = chunk_value<kFuseUp<BITS, XT>>(h2f((uint16_t)quad_bcast<2>(sv[t][c])), du,
+                                                            h2f((uint16_t)quad_bcast<3>(sv[t][c])), xs);
             pg[t] += on ? vg : 0.f;
             pu[t] += on ? vu : 0.f;
         }
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const float g = wave_sum_dpp(pg[t]), u = wave_sum_dpp(pu[t]);
+        const float g = wave_sum(pg[t]), u = wave_sum(pu[t]);
         if (lane == 0 && r0 + t < L.I) write_act(act, j, L.I, r0 + t, slot >= 0 ? silu_mul(g, u) : __builtin_nanf(""));
     }
 }
@@ -495,8 +512,8 @@ __global__ __launch_bounds__(64) void k_gate_up_generic(const Layer L, const voi
             x_to_f32<XT>(xr, xf);
             const float xs = chunk_sum_f32(xf);
             const int gidx = r * L.gpr_gu + (c * 32) / L.G;
-            pg += h2f(sc[gidx]) * chunk_dot_f32<BITS>(cg, xf) + h2f(mn[gidx]) * xs;
-            pu += h2f(sc[L.NGM + gidx]) * chunk_dot_f32<BITS>(cu, xf) + h2f(mn[L.NGM + gidx]) * xs;
+            pg += chunk_value<false>(h2f(sc[gidx]), chunk_dot_f32<BITS>(cg, xf), h2f(mn[gidx]), xs);
+            pu += chunk_value<kFuseUp<BITS, XT>>(h2f(sc[L.NGM + gidx]), chunk_dot_f32<BITS>(cu, xf), h2f(mn[L.NGM + gidx]), xs);
         }
         pg = wave_sum(pg);
         pu = wave_sum(pu);
@@ -614,7 +631,9 @@ __device__ __forceinline__ void down_rows(const Layer& L, const float* meta,
                     s_ = sv[t] & 0xFFFFu;
                     m_ = sv[t] >> 16;
                 }
-                const float v = h2f((uint16_t)s_) * d + h2f((uint16_t)m_) * as;
+                float v;
+                if constexpr (SPR_T == 0) v = chunk_value<false>(h2f((uint16_t)s_), d, h2f((uint16_t)m_), as);
+                else v = h2f((uint16_t)s_) * d + h2f((uint16_t)m_) * as;
                 p[t] = !ok ? __builtin_nanf("") : (row_ok ? v : 0.f);
             }
         }
@@ -847,14 +866,20 @@ __global__ __launch_bounds__(1024) void k_down_c2(const float* meta, const uint8
 // Kernel 2 for other shapes (weighted sum, G = 128 * 2^i, k * I / 32 <= 64 NC): k_down_rows' split. A wave computes
 // one whole output row over all k experts; lane l takes the (expert, chunk) pairs l, l + 64, ..., so all lanes work
 // whatever I / 32 is and no sum crosses waves. The activations of all experts are staged once per NWV rows, piece
-// i of chunk ch at i ^ (ch & 7) (the 8 lanes of a read phase hit 8 bank groups). 26.7 MB at H 4096,
-// I 1536, k = 8, 4 bits: 10.8 us with a wave per expert (k_down: 48 of 64 lanes at work, the activations staged per 4 rows)
-// and 9.4 here; at H 5120, I 1408, k = 10 49.1 us with k_down_generic and 16.6 here; two rows per wave spill at NC = 8.
-template <int BITS, int NC, int NWV>
+// i of chunk ch at i ^ (ch & 7) (the 8 lanes of a read phase hit 8 bank groups). The pairs' values then meet in the stage's
+// LDS, and each expert's are added, weighted and summed over the experts as the kernel that takes the shape otherwise does
+// it, so the bits are the same whatever the weights hold: WAVES in k_down's order (group_sum over 2^lsh_dn lanes, the products
+// rounded), else in k_down_generic's (the butterfly over 64 chunk columns, in rows of 16 lanes; fma). Bound by VALU
+// issue and, in the small shapes, by the chain of round trips. A layer (both kernels, 4 bits) of H 4096, I 1536, k = 8 takes
+// 22.9 us, 27.0 with the general kernels (k_down: a wave per expert, 48 of 64 lanes at work, the activations staged per 4
+// rows); H 5120, I 1408, k = 10 35.2 and 69.9; H 512, I 384, k = 8 6.7 and 7.7. Weighting each pair and summing the wave
+// once instead took 22.7, 34.5 and 6.0, in another order, and gave NaN for an infinite weight (0 times it in lanes without a
+// pair). Two rows per wave spill at NC = 8.
+template <int BITS, int NC, int NWV, bool WAVES>
 __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const uint8_t* __restrict__ pool,
                                                         int64_t slot_bytes, int nslots, int k,
                                                         const float* __restrict__ act, void* __restrict__ out,
-                                                        const Layer L) {
+                                                        const Layer L, int lsh_dn) {
     extern __shared__ uint4 stage4[];  // k * I / 4
     constexpr int APT = 64 * NC * 8 / (64 * NWV);
     const int lane = threadIdx.x & 63;
@@ -866,7 +891,7 @@ __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const
     const int h = rb * NWV + wv, hc = min(h, L.H - 1);
     const float inv = __builtin_amdgcn_rcpf((float)SPR);
     int ec[NC], sg[NC];
-    float fs[NC], fw[NC];
+    float fs[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int combo = min(lane + 64 * c, total - 1);
@@ -874,8 +899,10 @@ __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const
         sg[c] = combo - ec[c] * SPR;
         fs[c] = meta[ec[c]];
     }
+    const int lsh = WAVES ? lsh_dn : 4, EPR = 64 >> lsh, sub = lane & ((1 << lsh) - 1);
+    float wr[2];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) fw[c] = meta[k + ec[c]];
+    for (int r = 0; r < 2; ++r) wr[r] = meta[k + min(r * EPR + (lane >> lsh), k - 1)];
     const uint4* a4 = reinterpret_cast<const uint4*>(act);
     uint4 ap[APT];
 #pragma unroll
@@ -903,11 +930,10 @@ __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const
         stage4[ch * 8 + ((idx & 7) ^ (ch & 7))] = make_uint4(a.z, a.w, a.x, a.y);
     }
     __syncthreads();
-    float p = 0.f;
+    float p[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int ch = min(lane + 64 * c, total - 1);
-        const bool on = lane + 64 * c < total;
         float A[32];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -917,12 +943,96 @@ __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const
         }
         const float as = chunk_sum_f32(A);
         const float d = chunk_dot_f32<BITS>(cd[c], A);
-        const float v = h2f((uint16_t)(sv[c] & 0xFFFFu)) * d + h2f((uint16_t)(sv[c] >> 16)) * as;
-        p = __builtin_fmaf(fw[c], !on ? 0.f : okc[c] ? v : __builtin_nanf(""), p);
+        const float s = h2f((uint16_t)(sv[c] & 0xFFFFu)), m = h2f((uint16_t)(sv[c] >> 16));
+        const float v = chunk_value<!WAVES>(s, d, m, as);
+        p[c] = okc[c] ? v : __builtin_nanf("");
         __builtin_amdgcn_sched_barrier(0);  // one chunk's activations in registers at a time
     }
-    const float tot = wave_sum_dpp(p);
-    if (lane == 0 && h < L.H) store_out(out, L.odt, h, tot);
+    // beside the stage, or, past 64 KB with it, in its first NWV * total floats (of 32 total) once every wave has read it
+    if constexpr (NC > 6) __syncthreads();
+    float* part = reinterpret_cast<float*>(stage4 + (NC > 6 ? 0 : na)) + wv * total;
+    // lanes past the last pair repeat it (under a condition the compiler sank each chunk's arithmetic to its store, and held
+    // every chunk's activations until then)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) part[min(lane + 64 * c, total - 1)] = p[c];
+    wave_sync_lds();
+    // 2^lsh lanes sum an expert; two rounds of EPR experts at a time, their reads in flight together. What lies past a row
+    // or past the last expert adds +0 to sums that started at +0: no change, whatever they hold.
+    float acc = 0.f;
+    for (int e0 = 0; e0 < k; e0 += 2 * EPR) {
+        const bool two = e0 + EPR < k;
+        int e[2];
+        const float* pe[2];
+        float v[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            e[r] = e0 + r * EPR + (lane >> lsh);
+            pe[r] = part + min(e[r], k - 1) * SPR;
+            if (e0) wr[r] = meta[k + min(e[r], k - 1)];
+        }
+        if constexpr (WAVES) {  // group_sum's strided form
+            v[0] = v[1] = 0.f;
+            for (int i0 = sub; i0 - sub < SPR; i0 += 4 << lsh) {
+                float t[2][4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[0][u] = pe[0][min(i0 + (u << lsh), SPR - 1)];
+                if (two)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) t[1][u] = pe[1][min(i0 + (u << lsh), SPR - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[0] += i0 + (u << lsh) < SPR ? t[0][u] : 0.f;
+                if (two)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[1] += i0 + (u << lsh) < SPR ? t[1][u] : 0.f;
+            }
+            if (lsh >= 1) { v[0] += dpp_f<0xB1>(v[0]); v[1] += dpp_f<0xB1>(v[1]); }
+            if (lsh >= 2) { v[0] += dpp_f<0x4E>(v[0]); v[1] += dpp_f<0x4E>(v[1]); }
+            if (lsh >= 3) { v[0] += dpp_f<0x141>(v[0]); v[1] += dpp_f<0x141>(v[1]); }
+            if (lsh >= 4) { v[0] += dpp_f<0x140>(v[0]); v[1] += dpp_f<0x140>(v[1]); }
+        } else {  // wave_sum over 64 columns: steps 32 and 16 between a lane's four, then 8, 4, 2, 1 within the row
+            float s[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int i0 = sub; i0 - sub < SPR; i0 += 64) {
+                float t[2][4];
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) t[r][q] = pe[r][min(i0 + 16 * q, SPR - 1)];
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) s[r][q] += i0 + 16 * q < SPR ? t[r][q] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) v[r] = (s[r][0] + s[r][2]) + (s[r][1] + s[r][3]);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                v[r] += dpp_f<0x128>(v[r]);
+                v[r] += dpp_f<0x124>(v[r]);
+                v[r] += dpp_f<0x122>(v[r]);
+                v[r] += dpp_f<0x121>(v[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            wr[r] = e[r] < k ? wr[r] : 0.f;
+            v[r] = e[r] < k ? v[r] : 0.f;
+            if constexpr (WAVES) v[r] = wr[r] * v[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            for (int g = 0; g < EPR && e0 + r * EPR + g < k; g += 4)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float ve = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[r]), (g + u) << lsh));
+                    if constexpr (WAVES) {
+                        acc = add_rn(acc, ve);
+                    } else {
+                        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wr[r]), (g + u) << lsh));
+                        acc = __builtin_fmaf(w, ve, acc);
+                    }
+                }
+    }
+    if (lane == 0 && h < L.H) store_out(out, L.odt, h, acc);
 }
 
 // Kernel 2 (generic): any I, G and k; one workgroup of min(k, 16) waves per
@@ -954,7 +1064,7 @@ __global__ __launch_bounds__(1024) void k_down_generic(const Layer L, const floa
                     A[4 * i] = q.x; A[4 * i + 1] = q.y; A[4 * i + 2] = q.z; A[4 * i + 3] = q.w;
                 }
                 const int gidx = h * L.gpr_dn + (c * 32) / L.G;
-                v += h2f(sc[gidx]) * chunk_dot_f32<BITS>(cd, A) + h2f(mn[gidx]) * chunk_sum_f32(A);
+                v += chunk_value<true>(h2f(sc[gidx]), chunk_dot_f32<BITS>(cd, A), h2f(mn[gidx]), chunk_sum_f32(A));
             }
             v = wave_sum(v);
         } else {
@@ -970,7 +1080,7 @@ __global__ __launch_bounds__(1024) void k_down_generic(const Layer L, const floa
         __syncthreads();
         if (threadIdx.x == 0) {
             float acc = 0.f;
-            for (int jj = 0; jj < L.k; ++jj) acc += L.meta[L.k + jj] * rows[jj];
+            for (int jj = 0; jj < L.k; ++jj) acc = __builtin_fmaf(L.meta[L.k + jj], rows[jj], acc);
             store_out(out, L.odt, h, acc);
         }
     }
@@ -1116,13 +1226,20 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
     const int64_t pairs = (int64_t)L.k * L.spr_dn;
     // k_down_wide keeps every lane at work and needs no particular k; k_down stages a quarter of the activations per
     // row and stays where it can run (`waves`) with few output rows and many pairs: layers of 2,048 rows at k = 8 took
-    // 10.05 us with it against 10.35 (I 1024) and 11.6 against 12.0 (I 1408, k = 6), and 8.8 against 8.0 (I 1024, k = 5),
-    // 13.5 against 11.2 (3,072 rows, I 1152, k = 4) the other way. I = 768 keeps its tuned forms.
+    // 10.05 us with it against 10.35 (I 1024) and 11.6 against 12.0 (I 1408, k = 6), and 8.6 against 8.5 (I 1024, k = 5),
+    // 13.1 against 11.3 (3,072 rows, I 1152, k = 4) the other way. I = 768 keeps its tuned forms.
     if (WSUM && L.gsh >= 2 && pairs <= 512 && !(waves && (tuned || (L.H <= 2048 && pairs > 192)))) {
+        const int lsh = waves ? __builtin_ctz(lanes_per_sum(4 * (64 / L.spr_dn))) : 4;  // k_down sums 4 row iterations
         const bool n8 = L.H >= 4096;  // eight rows per staged activation once that still leaves two workgroups per CU
-#define WISP_DW(C, NWV)                                                                                               \
-    hipLaunchKernelGGL((k_down_wide<BITS, C, NWV>), dim3((L.H + NWV - 1) / NWV), dim3(64 * NWV), (size_t)pairs * 128, \
-                       st, L.meta, L.pool, L.slot_bytes, L.nslots, L.k, act, out, L)
+#define WISP_DWO(C, NWV, WV)                                                                                   \
+    hipLaunchKernelGGL((k_down_wide<BITS, C, NWV, WV>), dim3((L.H + NWV - 1) / NWV), dim3(64 * NWV),               \
+                       (size_t)pairs * (C > 6 ? 128 : 128 + 4 * NWV), st, L.meta, L.pool, L.slot_bytes, L.nslots,  \
+                       L.k, act, out, L, lsh)
+#define WISP_DW(C, NWV)                 \
+    do {                                \
+        if (waves) WISP_DWO(C, NWV, true); \
+        else WISP_DWO(C, NWV, false);   \
+    } while (0)
         if (pairs <= 64) WISP_DW(1, 4);
         else if (pairs <= 128) WISP_DW(2, 4);
         else if (pairs <= 192 && n8) WISP_DW(3, 8);
@@ -1131,9 +1248,11 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
         else if (pairs <= 256) WISP_DW(4, 4);
         else if (pairs <= 384 && n8) WISP_DW(6, 8);
         else if (pairs <= 384) WISP_DW(6, 4);
+        else if (pairs <= 448 && n8) WISP_DW(7, 8);
         else if (n8) WISP_DW(8, 8);
         else WISP_DW(8, 4);
 #undef WISP_DW
+#undef WISP_DWO
         return check_launch("k_down_wide");
     }
     if (!waves) {

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from wisp import kernels, quant
+from wisp import _lib, kernels, quant
 from wisp.cache import ExpertCache
 from wisp.moe import PagedMoEBlock, Runtime, route
 from wisp.store import ExpertStore
@@ -248,6 +248,44 @@ def test_block_runs_all_experts_at_once_where_the_cache_holds_them(nslots, n_sta
                                 rw.float().cpu().numpy(), H, I, bits)
         err = np.linalg.norm(y[0].double().cpu().numpy() - ref) / np.linalg.norm(ref)
         assert err <= 2.0**-8, (step, err)
+    for c in caches:
+        c.free()
+
+
+def test_block_pages_in_chunks_where_the_workspace_for_all_pairs_does_not_fit(monkeypatch):
+    """Memory that holds a chunk's workspace but not the one for all pairs: the block's prefill runs chunk by chunk, with
+    the bits and the bookkeeping of a block whose cache does not hold all experts at once."""
+    E, k, T, H, I, bits, n = 12, 4, 40, 256, 128, 4, 256 * 128
+    gen = torch.Generator(device=DEV).manual_seed(21)
+    store = ExpertStore(1, E, n, bits, 128)
+    store.fill(((e, torch.randn((3, n), generator=gen, device=DEV) * 0.05) for e in range(E)))
+    caches = [ExpertCache(store, E, policy="lru") for _ in range(2)]
+    gate = torch.nn.Linear(H, E, bias=False, device=DEV, dtype=torch.bfloat16)
+    cfg = SimpleNamespace(hidden_size=H, moe_intermediate_size=I, num_experts=E, num_experts_per_tok=k,
+                          norm_topk_prob=True)
+    blocks = [PagedMoEBlock(gate, 0, Runtime(store, c, chunk=5), cfg) for c in caches]
+    monkeypatch.setattr(caches[1], "holds_at_once", lambda n: False)
+    most, empty = _lib.lib().wisp_prefill_ws_bytes(T * k, H, I), torch.empty
+
+    def small(size, *a, **kw):
+        if kw.get("dtype") == torch.uint8 and size >= most:
+            raise torch.OutOfMemoryError("refused by the test")
+        return empty(size, *a, **kw)
+
+    for _ in range(2):
+        x = torch.randn((1, T, H), generator=gen, device=DEV).to(torch.bfloat16)
+        got = []
+        for refuse, block in ((True, blocks[0]), (False, blocks[1])):
+            with torch.no_grad(), monkeypatch.context() as m:
+                if refuse:
+                    m.setattr(kernels.torch, "empty", small)
+                y = block(x)
+            got.append(y[0] if isinstance(y, tuple) else y)
+        assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
+        a, b = caches[0].core, caches[1].core
+        assert a.stats == b.stats
+        assert [a.lookup(e) for e in range(E)] == [b.lookup(e) for e in range(E)]
+        assert blocks[0].rt.stats == blocks[1].rt.stats
     for c in caches:
         c.free()
 

@@ -245,7 +245,7 @@ _PLAN_IDS, _PLAN_ABSENT = 512, -(1 << 31)
 _PLAN_SEL = {torch.int64: 8, torch.int32: 4}
 
 
-def _plan_table(expert_slots):
+def plan_table(expert_slots):
     """{expert id: slot} as the GPU planner's int32 table (slot of id i), or None where it has no such form:
     an id outside [0, 512), or a slot that is no int32 or the mark of an absent expert."""
     try:
@@ -260,32 +260,62 @@ def _plan_table(expert_slots):
         return None
 
 
-def _plan_workspace(nbytes, dev):
+def _try_empty(shape, dtype, dev):
     try:
-        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        return torch.empty(shape, dtype=dtype, device=dev)
     except torch.OutOfMemoryError:
         return None
 
 
-def _prefill_routed(pool, table, x, sel, rw, H, I, bits, group, out, acc, max_pairs):
-    """The launches of a prefill whose routing (sel int64 or int32, rw of a float dtype, both contiguous) is in device
-    memory: the plan, the two GEMMs and the combine. False (nothing launched) where its workspace, which has room for
-    max_pairs whatever share of them the call runs, does not fit the free memory."""
+def _plan_workspace(nbytes, dev):
+    return _try_empty(nbytes, torch.uint8, dev)
+
+
+def prefill_planned(pool, x, sel, rw, n_ids, H, I, bits, group=128):
+    """moe_prefill in two steps, for a caller that can still choose another way: a function of the planner's slot table
+    (plan_table, of expert ids below n_ids) that launches the call and returns its result, or None, with nothing kept, where
+    the GPU planner does not take it or its workspace (for all T * k pairs) and output, allocated here, do not fit."""
+    _check_pool(pool)
+    _lib.require_gpu(pool, x, what="moe_prefill")
+    return _planned(pool, x.contiguous(), sel, rw, n_ids, H, I, bits, group, None)
+
+
+def _planned(pool, x, sel, rw, n_ids, H, I, bits, group, acc):
+    """prefill_planned of a checked pool and x (contiguous). The planner takes sel int64 or int32 on the GPU, rw of a float
+    dtype, and the shapes that the kernels take."""
     T, k = sel.shape
-    L = _lib.lib()
     dev = x.device
-    ws = _plan_workspace(L.wisp_prefill_routed_ws_bytes(T, k, max_pairs, len(table), H, I), dev)
+    if not (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k < 1 << 31 and k <= 32 and x.shape[0] >= T
+            and rw.numel() == T * k and rw.is_floating_point() and n_ids <= _PLAN_IDS and group == 128 and H % 256 == 0
+            and I % 128 == 0):
+        return None
+    if acc is not None:
+        assert acc.dtype == torch.float32 and acc.shape == (T, H) and acc.is_contiguous()
+    L = _lib.lib()
+    ws = _plan_workspace(L.wisp_prefill_routed_ws_bytes(T, k, T * k, n_ids, H, I), dev)
     if ws is None:
-        return False
-    _lib.check(
-        L.wisp_moe_prefill_routed(
-            _lib.ptr(pool), pool.stride(0), pool.shape[0], _lib.ptr(sel), _PLAN_SEL[sel.dtype], _lib.ptr(rw),
-            _X_DTYPES[rw.dtype], table.buffer_info()[0], len(table), max_pairs, _lib.ptr(x), T, k, H, I, bits, group,
-            _lib.ptr(ws), _lib.ptr(out), _lib.ptr(acc), _lib.stream(dev),
-        ),
-        "moe_prefill",
-    )
-    return True
+        return None
+    out = None
+    if acc is None:
+        out = _try_empty((T, H), torch.bfloat16, dev)
+        if out is None:
+            return None
+    s = sel.detach().contiguous()
+    w = rw.detach().reshape(-1).to(dev)
+    w = w.contiguous() if w.dtype in _X_DTYPES else w.to(torch.float32)
+
+    def launch(table):
+        _lib.check(
+            L.wisp_moe_prefill_routed(
+                _lib.ptr(pool), pool.stride(0), pool.shape[0], _lib.ptr(s), _PLAN_SEL[s.dtype], _lib.ptr(w),
+                _X_DTYPES[w.dtype], table.buffer_info()[0], len(table), T * k, _lib.ptr(x), T, k, H, I, bits, group,
+                _lib.ptr(ws), _lib.ptr(out), _lib.ptr(acc), _lib.stream(dev),
+            ),
+            "moe_prefill",
+        )
+        return acc if out is None else out
+
+    return launch
 
 
 def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=None):
@@ -306,22 +336,13 @@ def moe_prefill(pool, expert_slots, x, sel, rw, n, H, I, bits, group=128, acc=No
         raise TypeError(f"x must be bfloat16 (got {x.dtype})")
     x = x.contiguous()
     T, k = sel.shape
-    # the GPU planner's forms; every other one (ids past its table, odd dtypes and shapes, a workspace for all T * k pairs
-    # that does not fit, and what the kernels refuse) is planned on the host
-    if (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k < 1 << 31 and k <= 32 and x.shape[0] >= T
-            and rw.numel() == T * k and rw.is_floating_point() and expert_slots and group == 128 and H % 256 == 0
-            and I % 128 == 0):
-        table = _plan_table(expert_slots)
-        if table is not None:
-            if acc is None:
-                out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
-            else:
-                assert acc.dtype == torch.float32 and acc.shape == (T, H) and acc.is_contiguous()
-                out = None
-            w = rw.detach().reshape(-1).to(dev)
-            w = w.contiguous() if w.dtype in _X_DTYPES else w.to(torch.float32)
-            if _prefill_routed(pool, table, x, sel.detach().contiguous(), w, H, I, bits, group, out, acc, T * k):
-                return acc if out is None else out
+    # on the GPU where the planner takes the call; every other one (ids past its table, odd dtypes and shapes, a workspace
+    # for all T * k pairs that does not fit, and what the kernels refuse) is planned on the host
+    table = plan_table(expert_slots) if expert_slots else None
+    if table is not None:
+        launch = _planned(pool, x, sel, rw, len(table), H, I, bits, group, acc)
+        if launch is not None:
+            return launch(table)
     sel_cpu = sel.detach().cpu().numpy()
     experts = sorted(int(e) for e in expert_slots)
     order, tok, back, uniq, first, count = _prefill_plan(sel_cpu, experts, k)

@@ -185,7 +185,8 @@ class PagedMoEBlock(nn.Module):
     def _forward_dequant(self, x, rw, sel, pred, B, T, H):
         """Several tokens (moe.py:82-151, 'transfer' policy), experts paged in chunks of rt.chunk.
         4/3/2-bit experts with group 128: the grouped prefill kernels, once for all experts where
-        the cache keeps them all through the chunks' paging steps, else once per chunk (fp32
+        the cache keeps them all through the chunks' paging steps and the workspace for all pairs
+        fits the free memory, else once per chunk (fp32
         accumulation across chunks). Otherwise: per routed expert, dequantize its slot and run
         three bf16 GEMMs on its tokens."""
         rt, cache = self.rt, self.rt.cache
@@ -195,13 +196,16 @@ class PagedMoEBlock(nn.Module):
         keys = [base + int(e) for e in torch.unique(sel_cpu).tolist()]
         st = cache.store
         if st.bits in (2, 3, 4) and st.group == 128 and not cache.decode_on_load and x.dtype == torch.bfloat16:
-            from .kernels import moe_prefill
+            from .kernels import moe_prefill, plan_table, prefill_planned
 
-            if cache.holds_at_once(len(keys)):
-                # every routed expert stays resident through the chunks' paging steps: one set of launches for all
+            launch = None
+            if keys and cache.holds_at_once(len(keys)):
+                # every routed expert stays resident through the chunks' paging steps: one set of launches for all. Asked
+                # for before the paging: where the workspace for all pairs does not fit, the chunks need a part of it each
+                launch = prefill_planned(cache.gpu, x, sel, rw, keys[-1] - base + 1, H, self.I, st.bits, st.group)
+            if launch is not None:
                 slots = cache.ensure_chunks(keys, rt.chunk)
-                y = moe_prefill(cache.gpu, {kk - base: s for kk, s in zip(keys, slots)}, x, sel, rw, st.n, H, self.I,
-                                st.bits, st.group)
+                y = launch(plan_table({kk - base: s for kk, s in zip(keys, slots)}))
                 rt.stats["gpu_experts"] += len(keys)
                 if pred is not None:
                     self._prefetch_next(pred.cpu(), slots[(len(keys) - 1) // rt.chunk * rt.chunk :])

@@ -40,7 +40,7 @@ extern "C" {
 #define WISP_EINVAL (-1)
 #define WISP_EALIGN (-2)
 
-#define WISP_ABI_VERSION 2
+#define WISP_ABI_VERSION 3
 
 /* Float types of x and of the layer output (the reference kernels take any
  * float x and return x.dtype, wisp/kernels.py:132-137, 196-203, 315-322). */
@@ -205,12 +205,12 @@ int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, co
  * memory (no host synchronisation; capturable). sel: [T][k] expert ids, contiguous, int32 or int64 (sel_bytes 4 or 8);
  * rw: [T][k] routing weights of rw_dtype (WISP_DT_*); slot_of: HOST int32 [n_ids], read before the call returns: the
  * slot of expert id i, or INT32_MIN for an expert that this call does not run (its pairs, and those of ids outside
- * [0, n_ids), add nothing); at least one present, n_ids <= 512. max_pairs: at least the number of pairs of present
- * experts, T*k if unknown (with fewer the outputs are undefined; nothing is accessed out of bounds). ws:
- * wisp_prefill_routed_ws_bytes(T, k, max_pairs, n_ids, H, I), 256-byte aligned. Everything else as wisp_moe_prefill. */
-int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t max_pairs, int64_t n_ids, int64_t H, int64_t I);
+ * [0, n_ids), add nothing); at least one present, n_ids <= 512. ws: wisp_prefill_routed_ws_bytes(T, k, n_ids, H, I)
+ * (room for all T*k pairs, whatever share of them the call runs), 256-byte aligned. sel must not change while the call
+ * runs. Everything else as wisp_moe_prefill. */
+int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t n_ids, int64_t H, int64_t I);
 int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const void* sel, int sel_bytes,
-                            const void* rw, int rw_dtype, const int32_t* slot_of, int n_ids, int64_t max_pairs,
+                            const void* rw, int rw_dtype, const int32_t* slot_of, int n_ids,
                             const uint16_t* x, int T, int k, int64_t H, int64_t I, int bits, int64_t group, void* ws,
                             uint16_t* out, float* acc, void* stream);
 

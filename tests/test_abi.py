@@ -173,6 +173,41 @@ def test_prefill_argument_validation():
     assert L.wisp_prefill_ws_bytes(64, 2048, 768) == 64 * 768 * 2 + 64 * 2048 * 4
 
 
+def test_routed_prefill_argument_validation():
+    L = _lib.lib()
+    nb = 2506752
+    table = (ctypes.c_int32 * 600)(*range(600))
+    absent = (ctypes.c_int32 * 600)(*[-(1 << 31)] * 600)
+
+    def call(**kw):
+        a = dict(pool=FAKE, slot_bytes=nb, nslots=128, sel=FAKE, sel_bytes=8, rw=FAKE, rw_dtype=_lib.WISP_DT_BF16,
+                 slot_of=ctypes.cast(table, ctypes.c_void_p), n_ids=128, x=FAKE, T=8, k=8, H=2048, I=768, bits=4,
+                 group=128, ws=FAKE, out=FAKE, acc=None)
+        a.update(kw)
+        return L.wisp_moe_prefill_routed(*a.values(), None)
+
+    for bad in (dict(slot_of=None), dict(sel=None), dict(rw=None), dict(out=None), dict(sel_bytes=2), dict(rw_dtype=3),
+                dict(n_ids=0), dict(n_ids=513), dict(slot_of=ctypes.cast(absent, ctypes.c_void_p)), dict(group=64),
+                dict(H=2176, slot_bytes=nb * 2), dict(I=704), dict(bits=8), dict(k=33), dict(T=0),
+                dict(slot_bytes=nb - 16)):
+        assert call(**bad) == _lib.WISP_EINVAL, bad
+    for bad in (dict(x=ctypes.c_void_p(0x100002)), dict(ws=ctypes.c_void_p(0x100010)),
+                dict(out=ctypes.c_void_p(0x100004)), dict(out=None, acc=ctypes.c_void_p(0x100008))):
+        assert call(**bad) == _lib.WISP_EALIGN, bad
+    for bad in ((0, 8, 128, 2048, 768), (8, 0, 128, 2048, 768), (8, 8, 0, 2048, 768), (8, 8, 513, 2048, 768)):
+        assert L.wisp_prefill_routed_ws_bytes(*bad) == -1, bad
+    # the items (one per pair at most), tok and w, back, and the workspace of the GEMMs, each rounded to 256 bytes
+    assert L.wisp_prefill_routed_ws_bytes(8, 8, 128, 2048, 768) == 768 + 512 + 256 + L.wisp_prefill_ws_bytes(64, 2048, 768)
+
+
+def test_ensure_chunks_argument_validation():
+    L = _lib.lib()
+    keys = (ctypes.c_int64 * 4)(*range(4))
+    p = ctypes.cast(keys, ctypes.c_void_p)
+    for n, chunk, k, s in ((-1, 2, p, p), (4, 0, p, p), (4, 2, None, p), (4, 2, p, None)):
+        assert L.wisp_cache_ensure_chunks(FAKE, k, n, chunk, s, None) == _lib.WISP_EINVAL
+
+
 def test_decode_layer_argument_validation():
     """The graph decoder's dense kernels reject bad shapes and pointers before any launch."""
     L = _lib.lib()

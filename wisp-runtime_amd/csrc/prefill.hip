@@ -963,10 +963,10 @@ struct PlanTable {
 };
 struct PlanOut {
     int32_t* groups;  // [U][3]
-    int32_t* tok;     // [P]
-    float* w;         // [P]
+    int32_t* tok;     // [T * k]
+    float* w;         // [T * k]
     int32_t* back;    // [T][k]
-    int U, P, chunk;
+    int U, chunk;
 };
 
 __device__ __forceinline__ float plan_w(const void* rw, int rdt, int64_t i) {
@@ -1023,9 +1023,8 @@ __global__ __launch_bounds__(64 * kPlanWaves) void k_pf_plan(const ST* __restric
     int base = 0;  // this wave's first pair of the expert
     for (int i = 0; i < kPlanWaves; ++i) base += wless[i] + (i < wv ? wmine[i] : 0);
     auto place = [&](int p, int at) {
-        const bool room = b < nids && at < po.P;
-        po.back[p] = b == nids ? -1 : room ? at : po.P;
-        if (room) {
+        po.back[p] = b == nids ? -1 : at;
+        if (b < nids) {
             po.tok[at] = p / k;
             po.w[at] = plan_w(rw, rdt, p);
         }
@@ -1077,11 +1076,9 @@ __global__ __launch_bounds__(64 * kPlanWaves) void k_pf_plan(const ST* __restric
         for (int i = 0; i <= nf; ++i) {
             const int u = i < nf ? uf + i : ul, p0 = first + i * 16 * full;
             const int cnt = i < nf ? 16 * full : c - nf * 16 * full;
-            if (u < po.U) {
-                po.groups[3 * u] = slots[tid];
-                po.groups[3 * u + 1] = min(p0, po.P);
-                po.groups[3 * u + 2] = max(0, min(cnt, po.P - p0));
-            }
+            po.groups[3 * u] = slots[tid];
+            po.groups[3 * u + 1] = p0;
+            po.groups[3 * u + 2] = cnt;
         }
     }
     for (int u = used + tid; u < po.U; u += 64 * kPlanWaves)  // past the last item: no pairs
@@ -1232,17 +1229,18 @@ static int plan_chunk(int64_t pairs, int64_t present) {
 }
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
-extern "C" int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t max_pairs, int64_t n_ids, int64_t H, int64_t I) {
-    if (T < 1 || k < 1 || max_pairs < 1 || max_pairs > T * k || n_ids < 1 || n_ids > kPlanIds || H < 1 || I < 1) return -1;
-    return up256(12 * plan_items(max_pairs, n_ids, 16)) + up256(8 * max_pairs) + up256(4 * T * k) +
-           wisp_prefill_ws_bytes(max_pairs, H, I);
+extern "C" int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t n_ids, int64_t H, int64_t I) {
+    if (T < 1 || k < 1 || n_ids < 1 || n_ids > kPlanIds || H < 1 || I < 1) return -1;
+    const int64_t pairs = T * k;
+    return up256(12 * plan_items(pairs, n_ids, 16)) + up256(8 * pairs) + up256(4 * pairs) +
+           wisp_prefill_ws_bytes(pairs, H, I);
 }
 
 // moe.py:82-151: the grouping of the (token, expert) pairs and wisp_moe_prefill, from the routing in device memory
 extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, const void* sel,
                                        int sel_bytes, const void* rw, int rw_dtype, const int32_t* slot_of, int n_ids,
-                                       int64_t max_pairs, const uint16_t* x, int T, int k, int64_t H, int64_t I, int bits,
-                                       int64_t group, void* ws, uint16_t* out, float* acc, void* stream) {
+                                       const uint16_t* x, int T, int k, int64_t H, int64_t I, int bits, int64_t group,
+                                       void* ws, uint16_t* out, float* acc, void* stream) {
     clear_error();
     if (!pool || !sel || !rw || !slot_of || !x || !ws || (!out && !acc)) return fail_inval("null pointer");
     if (sel_bytes != 4 && sel_bytes != 8) return fail_inval("sel must be int32 or int64");
@@ -1250,7 +1248,8 @@ extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, 
         return fail_inval("rw_dtype must be WISP_DT_BF16, WISP_DT_F16 or WISP_DT_F32");
     if (n_ids < 1 || n_ids > kPlanIds) return fail_inval("n_ids must be in [1, 512]");
     if ((int64_t)T * k >= (int64_t)1 << 31) return fail_inval("T*k must be below 2^31");
-    const int rc = prefill_check(pool, slot_bytes, nslots, x, T, k, max_pairs, H, I, bits, group, ws, out, acc);
+    const int64_t pairs = (int64_t)T * k;
+    const int rc = prefill_check(pool, slot_bytes, nslots, x, T, k, pairs, H, I, bits, group, ws, out, acc);
     if (rc) return rc;
     PlanTable tb;
     int64_t present = 0;
@@ -1260,17 +1259,16 @@ extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, 
     }
     if (!present) return fail_inval("no expert in slot_of");
     PlanOut po;
-    po.chunk = plan_chunk(max_pairs, present);
-    po.U = (int)plan_items(max_pairs, present, po.chunk);
-    po.P = (int)max_pairs;
+    po.chunk = plan_chunk(pairs, present);
+    po.U = (int)plan_items(pairs, present, po.chunk);
     uint8_t* at = static_cast<uint8_t*>(ws);
     po.groups = reinterpret_cast<int32_t*>(at);
-    at += up256(12 * plan_items(max_pairs, n_ids, 16));
+    at += up256(12 * plan_items(pairs, n_ids, 16));
     po.tok = reinterpret_cast<int32_t*>(at);
-    po.w = reinterpret_cast<float*>(at + 4 * max_pairs);
-    at += up256(8 * max_pairs);
+    po.w = reinterpret_cast<float*>(at + 4 * pairs);
+    at += up256(8 * pairs);
     po.back = reinterpret_cast<int32_t*>(at);
-    at += up256(4 * (int64_t)T * k);
+    at += up256(4 * pairs);
     hipStream_t st = (hipStream_t)stream;
     if (sel_bytes == 8)
         hipLaunchKernelGGL(k_pf_plan<int64_t>, dim3(n_ids + 1), dim3(64 * kPlanWaves), 0, st, (const int64_t*)sel, rw,
@@ -1282,6 +1280,6 @@ extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, 
     F.groups = po.groups;
     F.tok = po.tok;
     F.w = po.w;
-    return prefill_launch(F, pool, slot_bytes, nslots, po.U, std::min(po.chunk, T), po.back, false, max_pairs, x, T, k, H, I,
+    return prefill_launch(F, pool, slot_bytes, nslots, po.U, std::min(po.chunk, T), po.back, false, pairs, x, T, k, H, I,
                           bits, at, out, acc, st);
 }

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(PKG_ROOT, "lib", "libwisp_hip.so")
-ABI_VERSION = 2
+ABI_VERSION = 3
 
 WISP_OK, WISP_EINVAL, WISP_EALIGN = 0, -1, -2
 WISP_DT_BF16, WISP_DT_F16, WISP_DT_F32 = 0, 1, 2
@@ -47,8 +47,8 @@ SIGNATURES = {
     "wisp_prefill_ws_bytes": (_i64, [_i64, _i64, _i64]),
     "wisp_moe_prefill": (_i32, [_vp, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _vp, _i32, _i32, _i64, _i64,
                                 _i32, _i64, _vp, _vp, _vp, _vp]),
-    "wisp_prefill_routed_ws_bytes": (_i64, [_i64, _i32, _i64, _i64, _i64, _i64]),
-    "wisp_moe_prefill_routed": (_i32, [_vp, _i64, _i64, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _vp, _i32, _i32, _i64, _i64,
+    "wisp_prefill_routed_ws_bytes": (_i64, [_i64, _i32, _i64, _i64, _i64]),
+    "wisp_moe_prefill_routed": (_i32, [_vp, _i64, _i64, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i32, _i64, _i64,
                                        _i32, _i64, _vp, _vp, _vp, _vp]),
     "wisp_mxfp4_to_bf16": (_i32, [_vp, _vp, _i64, _vp, _vp]),
     "wisp_dl_gemv": (_i32, [_vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp,

@@ -292,7 +292,7 @@ def _planned(pool, x, sel, rw, n_ids, H, I, bits, group, acc):
     if acc is not None:
         assert acc.dtype == torch.float32 and acc.shape == (T, H) and acc.is_contiguous()
     L = _lib.lib()
-    ws = _plan_workspace(L.wisp_prefill_routed_ws_bytes(T, k, T * k, n_ids, H, I), dev)
+    ws = _plan_workspace(L.wisp_prefill_routed_ws_bytes(T, k, n_ids, H, I), dev)
     if ws is None:
         return None
     out = None
@@ -308,7 +308,7 @@ def _planned(pool, x, sel, rw, n_ids, H, I, bits, group, acc):
         _lib.check(
             L.wisp_moe_prefill_routed(
                 _lib.ptr(pool), pool.stride(0), pool.shape[0], _lib.ptr(s), _PLAN_SEL[s.dtype], _lib.ptr(w),
-                _X_DTYPES[w.dtype], table.buffer_info()[0], len(table), T * k, _lib.ptr(x), T, k, H, I, bits, group,
+                _X_DTYPES[w.dtype], table.buffer_info()[0], len(table), _lib.ptr(x), T, k, H, I, bits, group,
                 _lib.ptr(ws), _lib.ptr(out), _lib.ptr(acc), _lib.stream(dev),
             ),
             "moe_prefill",

@@ -205,7 +205,7 @@ int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t nslots, co
  * memory (no host synchronisation; capturable). sel: [T][k] expert ids, contiguous, int32 or int64 (sel_bytes 4 or 8);
  * rw: [T][k] routing weights of rw_dtype (WISP_DT_*); slot_of: HOST int32 [n_ids], read before the call returns: the
  * slot of expert id i, or INT32_MIN for an expert that this call does not run (its pairs, and those of ids outside
- * [0, n_ids), add nothing); at least one present, n_ids <= 512. ws: wisp_prefill_routed_ws_bytes(T, k, n_ids, H, I)
+ * [0, n_ids), add nothing); at least one present, n_ids <= 512; T*k <= 2^30. ws: wisp_prefill_routed_ws_bytes(T, k, n_ids, H, I)
  * (room for all T*k pairs, whatever share of them the call runs), 256-byte aligned. sel must not change while the call
  * runs. Everything else as wisp_moe_prefill. */
 int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t n_ids, int64_t H, int64_t I);

@@ -194,6 +194,10 @@ def test_routed_prefill_argument_validation():
     for bad in (dict(x=ctypes.c_void_p(0x100002)), dict(ws=ctypes.c_void_p(0x100010)),
                 dict(out=ctypes.c_void_p(0x100004)), dict(out=None, acc=ctypes.c_void_p(0x100008))):
         assert call(**bad) == _lib.WISP_EALIGN, bad
+    # the plan's counters are 32-bit and step past the last pair
+    assert call(T=(1 << 26) + 1, k=16) == _lib.WISP_EINVAL and b"T*k" in L.wisp_last_error()
+    assert L.wisp_prefill_routed_ws_bytes((1 << 26) + 1, 16, 128, 2048, 768) == -1
+    assert L.wisp_prefill_routed_ws_bytes(1 << 26, 16, 128, 256, 128) > 0
     for bad in ((0, 8, 128, 2048, 768), (8, 0, 128, 2048, 768), (8, 8, 0, 2048, 768), (8, 8, 513, 2048, 768)):
         assert L.wisp_prefill_routed_ws_bytes(*bad) == -1, bad
     # the items (one per pair at most), tok and w, back, and the workspace of the GEMMs, each rounded to 256 bytes

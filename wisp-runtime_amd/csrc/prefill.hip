@@ -956,6 +956,7 @@ __global__ __launch_bounds__(256) void k_pf_combine(const float* __restrict__ y,
 // reads it, from L2): and by the ballots' issue: 5.1 us for 64 tokens, 18 for
 // 4,096 (8 experts each); the grouping in numpy and its uploads took about 100 and 1,600 us, after a wait for the GPU.
 // ===========================================================================
+constexpr int64_t kPlanPairs = (int64_t)1 << 30;  // the pair indices stay in 32 bits, with the steps that run past the last
 constexpr int kPlanIds = 512, kPlanWaves = 16, kPlanList = 256;
 constexpr int32_t kPlanAbsent = INT32_MIN;
 struct PlanTable {
@@ -1230,7 +1231,7 @@ static int plan_chunk(int64_t pairs, int64_t present) {
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
 extern "C" int64_t wisp_prefill_routed_ws_bytes(int64_t T, int k, int64_t n_ids, int64_t H, int64_t I) {
-    if (T < 1 || k < 1 || n_ids < 1 || n_ids > kPlanIds || H < 1 || I < 1) return -1;
+    if (T < 1 || k < 1 || T > kPlanPairs / k || n_ids < 1 || n_ids > kPlanIds || H < 1 || I < 1) return -1;
     const int64_t pairs = T * k;
     return up256(12 * plan_items(pairs, n_ids, 16)) + up256(8 * pairs) + up256(4 * pairs) +
            wisp_prefill_ws_bytes(pairs, H, I);
@@ -1247,8 +1248,8 @@ extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, 
     if (rw_dtype != WISP_DT_BF16 && rw_dtype != WISP_DT_F16 && rw_dtype != WISP_DT_F32)
         return fail_inval("rw_dtype must be WISP_DT_BF16, WISP_DT_F16 or WISP_DT_F32");
     if (n_ids < 1 || n_ids > kPlanIds) return fail_inval("n_ids must be in [1, 512]");
-    if ((int64_t)T * k >= (int64_t)1 << 31) return fail_inval("T*k must be below 2^31");
     const int64_t pairs = (int64_t)T * k;
+    if (pairs > kPlanPairs) return fail_inval("T*k must be at most 2^30");
     const int rc = prefill_check(pool, slot_bytes, nslots, x, T, k, pairs, H, I, bits, group, ws, out, acc);
     if (rc) return rc;
     PlanTable tb;

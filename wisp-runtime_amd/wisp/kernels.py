@@ -241,7 +241,7 @@ def _prefill_chunks(uniq, first, count, chunk=None):
     return ex[o], start[o], cnt[o]
 
 
-_PLAN_IDS, _PLAN_ABSENT = 512, -(1 << 31)
+_PLAN_IDS, _PLAN_PAIRS, _PLAN_ABSENT = 512, 1 << 30, -(1 << 31)
 _PLAN_SEL = {torch.int64: 8, torch.int32: 4}
 
 
@@ -285,7 +285,7 @@ def _planned(pool, x, sel, rw, n_ids, H, I, bits, group, acc):
     dtype, and the shapes that the kernels take."""
     T, k = sel.shape
     dev = x.device
-    if not (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k < 1 << 31 and k <= 32 and x.shape[0] >= T
+    if not (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k <= _PLAN_PAIRS and k <= 32 and x.shape[0] >= T
             and rw.numel() == T * k and rw.is_floating_point() and n_ids <= _PLAN_IDS and group == 128 and H % 256 == 0
             and I % 128 == 0):
         return None

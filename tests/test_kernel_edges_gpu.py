@@ -190,6 +190,18 @@ def test_prefill_is_planned_on_the_host_where_the_workspace_does_not_fit(monkeyp
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("on", ["cpu", DEV])
+def test_prefill_of_a_width_without_kernels_where_no_pair_runs(on):
+    """A call none of whose pairs has an expert is zeros, whatever its width: nothing is launched for it."""
+    H, I, n = 256, 128, 256 * 128
+    pool = torch.zeros((2, quant.expert_nbytes(n, 8, 128)), dtype=torch.uint8, device=DEV)
+    x = torch.ones((3, H), dtype=torch.bfloat16, device=DEV)
+    sel, rw = torch.full((3, 2), 9, device=on), torch.ones((3, 2), device=DEV)
+    assert (kernels.moe_prefill(pool, {0: 0, 1: 1}, x, sel, rw, n, H, I, 8) == 0).all()
+    with pytest.raises(ValueError):
+        kernels.moe_prefill(pool, {9: 0}, x, sel, rw, n, H, I, 8)
+
+
 def test_prefill_under_graph_capture_follows_the_routing():
     E, k, T, H, I, bits, n = 8, 2, 70, 256, 128, 4, 256 * 128
     rng = np.random.default_rng(5)

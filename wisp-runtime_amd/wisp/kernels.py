@@ -286,7 +286,7 @@ def _planned(pool, x, sel, rw, n_ids, H, I, bits, group, acc):
     T, k = sel.shape
     dev = x.device
     if not (sel.device == dev and sel.dtype in _PLAN_SEL and 0 < T * k <= _PLAN_PAIRS and k <= 32 and x.shape[0] >= T
-            and rw.numel() == T * k and rw.is_floating_point() and n_ids <= _PLAN_IDS and group == 128 and H % 256 == 0
+            and rw.numel() == T * k and rw.is_floating_point() and n_ids <= _PLAN_IDS and bits in (2, 3, 4) and group == 128 and H % 256 == 0
             and I % 128 == 0):
         return None
     if acc is not None:

@@ -139,8 +139,7 @@ def _routing(gen, T, E, k):
     return sel, rw.to(torch.bfloat16)
 
 
-# the plan formed on the GPU against the host's, bit for bit: one token, runs that are not whole waves, a hot expert
-# (more matches in a wave's run than its list holds), every chunk size, the largest table, k = 32 (the wide combine)
+# the plan formed on the GPU against the host's, bit for bit: one token, runs that are not whole waves, every chunk size, the largest table, k = 32 (the wide combine)
 @pytest.mark.parametrize("E,k,T,bits", [(6, 2, 1, 4), (6, 2, 17, 3), (4, 2, 900, 4), (300, 8, 50, 2), (512, 4, 40, 4),
                                         (40, 32, 33, 4), (3, 1, 9000, 4), (5, 3, 333, 3)])
 @pytest.mark.parametrize("mode", ["all", "part", "twice", "outside"])
@@ -169,6 +168,26 @@ def test_prefill_plan_on_the_gpu_equals_the_hosts(E, k, T, bits, mode):
     kernels.moe_prefill(pool, slots, x, s32, rw, n, H, I, bits, acc=acc)
     kernels.moe_prefill(pool, slots, x, s32.cpu(), rw, n, H, I, bits, acc=ref)
     assert torch.equal(acc.view(torch.int32), ref.view(torch.int32))
+
+
+# a hot expert has more matches in a wave's run of the pairs than its list of 256 holds: they are read again and placed by
+# their ranks. Runs of 576 pairs (the last one partial) and of 1,088; all pairs of one expert, most, and two such experts
+@pytest.mark.parametrize("T,k", [(9000, 1), (8640 + 33, 2), (8191, 1)])
+@pytest.mark.parametrize("share", [1.0, 0.9, 0.5])
+def test_prefill_plan_of_a_hot_expert(T, k, share):
+    E, H, I, bits, n = 5, 256, 128, 4, 256 * 128
+    rng = np.random.default_rng(T + k)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(E)])).to(DEV)
+    hot = rng.random(T) < share
+    sel = np.stack([np.where(hot, 3, 1), np.where(hot, rng.integers(4, 6, T), 0)], 1)[:, :k]  # 5: an absent expert
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16).to(DEV)
+    rw = torch.from_numpy(rng.random((T, k)).astype(np.float32)).to(DEV)
+    st = torch.from_numpy(np.ascontiguousarray(sel))
+    slots = {e: (e + 2) % E for e in range(E)}
+    got = kernels.moe_prefill(pool, slots, x, st.to(DEV), rw, n, H, I, bits)
+    want = kernels.moe_prefill(pool, slots, x, st, rw, n, H, I, bits)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
 def test_prefill_is_planned_on_the_host_where_the_workspace_does_not_fit(monkeypatch):

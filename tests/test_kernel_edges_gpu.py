@@ -170,6 +170,25 @@ def test_prefill_plan_on_the_gpu_equals_the_hosts(E, k, T, bits, mode):
     assert torch.equal(acc.view(torch.int32), ref.view(torch.int32))
 
 
+# skewed routing, and the item sizes of a card that the experts' rows fill (by the parity of I / 128 and the width) and of
+# one that they do not: the outputs do not depend on them
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("E,I,T", [(400, 128, 100), (400, 128, 700), (200, 256, 60), (200, 256, 500), (40, 256, 300)])
+def test_prefill_plan_of_skewed_routing(bits, E, I, T):
+    H, k, n = 256, 4, 256 * I
+    rng = np.random.default_rng(E + T + bits)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(5)])).to(DEV)
+    key = -1.1 * np.log(np.arange(1, E + 1)) + rng.gumbel(size=(T, E))  # k different experts of a Zipf(1.1) draw
+    sel = torch.from_numpy(rng.permutation(E)[np.argsort(-key, 1)[:, :k]].astype(np.int64))
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16).to(DEV)
+    rw = torch.from_numpy(rng.random((T, k)).astype(np.float32)).to(DEV)
+    slots = {e: e % 5 for e in range(E)}
+    got = kernels.moe_prefill(pool, slots, x, sel.to(DEV), rw, n, H, I, bits)
+    want = kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 # a hot expert has more matches in a wave's run of the pairs than its list of 256 holds: they are read again and placed by
 # their ranks. Runs of 576 pairs (the last one partial) and of 1,088; all pairs of one expert, most, and two such experts
 @pytest.mark.parametrize("T,k", [(9000, 1), (8640 + 33, 2), (8191, 1)])

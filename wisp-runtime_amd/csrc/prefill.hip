@@ -1221,12 +1221,23 @@ extern "C" int wisp_moe_prefill(const uint8_t* pool, int64_t slot_bytes, int64_t
 static int64_t plan_items(int64_t pairs, int64_t present, int chunk) {
     return std::max<int64_t>(1, std::min(pairs, present + pairs / chunk));
 }
-// Pairs per work item: the smallest of 16, 32, 64 and 128 that the mean of an expert's pairs plus two of its
-// (Poisson) deviations fits. Fewer tiles per pass leave more workgroups per CU, and items that are split read their
-// expert's rows twice. The outputs do not depend on it.
-static int plan_chunk(int64_t pairs, int64_t present) {
+// Pairs per work item. An expert of more pairs is split, and each item reads and dequantizes its rows again; fewer tiles
+// per pass leave more workgroups per CU, and a split hot expert spreads over an idle chip. So: the smallest of 16, 32, 64
+// and 128 that the mean of an expert's pairs plus two of its (Poisson) deviations fits; but where the experts' rows fill
+// the card anyhow (three workgroups of 64 activation rows on each of 256 CUs), at least 64, whatever the skew of the
+// routing, and 32 where the down GEMM is in its register form. 2-bit rows of less than 4,096 values keep the 16: their
+// short passes want the workgroups. us a call, uniform / Zipf(1.1) routing, by the mean alone -> by this:
+// 2048 x 768, 128 experts, top-8, 333 tokens 104.2 / 115.2 -> 101.8 / 114.0 at 4 bits, 109.3 / 121.1 -> 105.1 / 115.4 at 3;
+// 128 tokens at 3 bits 95.2 / 103.7 -> 91.6 / 94.9; 4096 x 1536, 64 experts, top-4, 64 tokens 147.6 / 128.3 -> 148.9 / 121.2,
+// 333 183.2 / 213.2 -> 175.9 / 193.0; 2048 x 1408, 64 experts, top-6, 64 tokens 86.7 / 91.1 -> 83.5 / 81.6; the other way
+// 32 tokens over the first 77.2 / 57.3 -> 76.7 / 60.2. 64 at 2 bits there: 128 uniform tokens 74.6 -> 78.5. A card that is
+// not full: 3072 x 1152, 32 experts, top-2, 250 tokens by the mean 70.1 / 70.7, 128 pairs an item 73.3 / 87.1. The outputs
+// do not depend on it.
+static int plan_chunk(int64_t pairs, int64_t present, int64_t H, int64_t I, int bits) {
     const double mean = (double)pairs / (double)std::max<int64_t>(1, present), most = mean + 2 * std::sqrt(mean);
-    return most <= 16 ? 16 : most <= 32 ? 32 : most <= 64 ? 64 : 128;
+    const int by_mean = most <= 16 ? 16 : most <= 32 ? 32 : most <= 64 ? 64 : 128;
+    if (std::min(pairs, present) * (I / 64) < 3 * 256 || (bits == 2 && H < 4096 && by_mean == 16)) return by_mean;
+    return std::max(by_mean, I / 128 % 2 ? 32 : 64);
 }
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
@@ -1260,7 +1271,7 @@ extern "C" int wisp_moe_prefill_routed(const uint8_t* pool, int64_t slot_bytes, 
     }
     if (!present) return fail_inval("no expert in slot_of");
     PlanOut po;
-    po.chunk = plan_chunk(pairs, present);
+    po.chunk = plan_chunk(pairs, present, H, I, bits);
     po.U = (int)plan_items(pairs, present, po.chunk);
     uint8_t* at = static_cast<uint8_t*>(ws);
     po.groups = reinterpret_cast<int32_t*>(at);

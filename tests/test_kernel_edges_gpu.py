@@ -73,6 +73,25 @@ def test_attn_decode_wide_merge(Hq, Hk, D):
         assert ((got - ref).norm() / ref.norm()).item() <= 2.0**-8, pos
 
 
+# a short context in a large cache merges as in a small one, bit for bit: up to 128 chunks by four waves
+@pytest.mark.parametrize("Hq,Hk,D", [(8, 2, 128), (4, 2, 64), (2, 2, 256)])
+def test_attn_decode_short_context_in_a_large_cache(Hq, Hk, D):
+    gen = torch.Generator(device=DEV).manual_seed(Hq + D)
+    q, k, v = (torch.randn(s, generator=gen, device=DEV).to(torch.bfloat16)
+               for s in ((1, Hq, 1, D), (1, Hk, 8192 + 64, D), (1, Hk, 8192 + 64, D)))
+    ks, vs = k[:, :, :8192].contiguous(), v[:, :, :8192].contiguous()
+    for pos in (0, 64, 4031, 4095, 4096, 4160, 8127, 8128, 8191):
+        p = torch.tensor([pos], device=DEV)
+        got, want = kernels.attn_decode(q, k, v, p, D**-0.5), kernels.attn_decode(q, ks, vs, p, D**-0.5)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), pos
+    # one chunk more: all eight waves
+    got = kernels.attn_decode(q, k, v, torch.tensor([8192], device=DEV), D**-0.5).view(Hq, D).double()
+    kk, vv = (t[0, :, :8193].double().repeat_interleave(Hq // Hk, 0) for t in (k, v))
+    w = ((kk @ q[0, :, 0].double()[:, :, None])[..., 0] * D**-0.5).softmax(-1)
+    ref = (w[:, None] @ vv)[:, 0]
+    assert ((got - ref).norm() / ref.norm()).item() <= 2.0**-8  # one bf16 rounding and fp32 sums
+
+
 # kernel 1 rows of 2, 3 and 4 chunks per lane (a remainder in each; float32 x of four goes to the generic kernel),
 # kernel 2 with 4 to 512 (expert, chunk) pairs: part of one step, every step count, and more than 16 experts
 @pytest.mark.parametrize("bits", [4, 3, 2])

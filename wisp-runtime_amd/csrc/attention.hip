@@ -20,6 +20,8 @@
 // the two launches' dependent round trips dominate.
 #include <math.h>
 
+#include <type_traits>
+
 #include "wisp_device.hpp"
 #include "wisp_internal.hpp"
 
@@ -297,8 +299,8 @@ __device__ __forceinline__ float row0_max(float v) {
 }
 
 // One workgroup (NW = 4 or 8 waves) per query head: wave w < 4 merges chunks w, w+4, ...
-// of the first 64 in a batch of 16, and wave w < NW chunks 64 + w, 64 + w + NW, ... in
-// batches of 16, with a running maximum. Lane b < 16 reads the m and l of the batch's
+// of the first 64 in a batch of 16, and, past 128 chunks, wave w < NW chunks 64 + w,
+// 64 + w + NW, ... in batches of 16 (up to 128 the lower four go on), with a running maximum. Lane b < 16 reads the m and l of the batch's
 // chunk b and computes its weight (one exponential per chunk); the weights reach the
 // o sums of every lane through readlane. The waves' sums are rescaled to the
 // common maximum in LDS. Only the chunks up to pos have records (pos read from device
@@ -322,11 +324,11 @@ __global__ __launch_bounds__(64 * NW) void k_attn_merge(const float* __restrict_
     // (stale or never written) are masked once it has arrived -- never multiplied, so their
     // bits cannot reach the sums. The first batch always exists (chunk 0).
     // Waves 4 .. NW - 1 take no part in the first 64 chunks: they wait for the position, then all NW waves share
-    // the chunks from 64 on.
+    // the chunks from 64 on, where there are more than the lower four take in one more batch.
     int c0 = 0, nv, sw = 4;  // the batch: chunks c0 + wv + sw * b
     if (NW > 4 && wv >= 4) {
         nv = (int)min<int64_t>(nsplit, pos / kChunk + 1);
-        c0 = 4 * B;
+        c0 = nv > 8 * B ? 4 * B : nv;
         sw = NW;
     } else {
         nv = 1;
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_merge(const float* __restrict_
         }
         M = Mn;
         c0 += sw * B;
-        sw = NW;
+        sw = nv > 8 * B ? NW : 4;
     }
     if (lane == 0) {
         red_m[wv] = M;
@@ -374,16 +376,22 @@ __global__ __launch_bounds__(64 * NW) void k_attn_merge(const float* __restrict_
     __syncthreads();
     if (threadIdx.x < D) {
         const int d = threadIdx.x;
-        float Mx = red_m[0];  // finite: chunk 0 exists
+        float v, Lt;
+        auto add_up = [&](auto n) {
+            float Mx = red_m[0];  // finite: chunk 0 exists
 #pragma unroll
-        for (int w = 1; w < NW; ++w) Mx = fmaxf(Mx, red_m[w]);
-        float v = 0.f, Lt = 0.f;
+            for (int w = 1; w < n; ++w) Mx = fmaxf(Mx, red_m[w]);
+            v = Lt = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float f = red_m[w] == -INFINITY ? 0.f : expf(red_m[w] - Mx);
-            v += f * red_o[w][d];
-            Lt += f * red_l[w];
-        }
+            for (int w = 0; w < n; ++w) {
+                const float f = red_m[w] == -INFINITY ? 0.f : expf(red_m[w] - Mx);
+                v += f * red_o[w][d];
+                Lt += f * red_l[w];
+            }
+        };
+        // up to 128 chunks: waves 4 .. NW - 1 had none
+        if (NW > 4 && pos / kChunk >= 8 * B) add_up(std::integral_constant<int, NW>{});
+        else add_up(std::integral_constant<int, 4>{});
         out[(int64_t)h * D + d] = f32_to_bf16(v / Lt);
     }
 }
@@ -401,7 +409,8 @@ static void launch_attn(const uint16_t* q, const uint16_t* kc, const uint16_t* v
     // The capacity decides (the position is on the device). A head's four waves walk its records 64 at a time, one
     // round trip each: 11.0 us of merge at 512 records, 7.6 with eight waves (32 / 4 heads of 128, 32k positions: 26.5
     // -> 23.1 us per call; 9,000 positions 12.8 -> 11.9; sixteen waves 23.3 and 13.0). Where a large cache is still
-    // short the second four waves cost 0.3 us (7.55 -> 7.83 us at 4,090 positions).
+    // short (up to 128 chunks) the second four waves have no chunk and the last sum leaves them out: 9.67 -> 9.73 us a
+    // call at 4,090 positions, 11.15 -> 11.17 at 6,000 (9.96 and 11.35 with their empty sums added).
     if (nsplit > kMergeWide)
         hipLaunchKernelGGL((k_attn_merge<D, 8>), dim3(hk * G), dim3(512), 0, st, part, pos, G, nsplit, out);
     else

@@ -378,3 +378,34 @@ def test_prefill_dma_every_width(bits, E, H, I, T, k):
         # the oracle's activation is rounded to bf16 as the kernels' is; one more rounding of the result
         err = np.linalg.norm(got.double().cpu().numpy() - ref) / np.linalg.norm(ref)
         assert err <= 2.0**-8, (on, err)
+
+
+# x of 2 GiB: gate_up in its register form (scales staged in LDS up to 16 K groups, read as needed past them), against the
+# halves of the tokens, whose x the LDS-DMA form takes: the same bits. 3 experts, one of them without a slot
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("H,I", [(2048, 256), (4096, 128)])
+def test_prefill_of_two_gib_of_tokens(bits, H, I):
+    n, T = H * I, (1 << 30) // H
+    rng = np.random.default_rng(H + bits)
+    pool = torch.from_numpy(np.stack([O.quantize((rng.standard_normal(3 * n) * 0.05).astype(np.float32), bits, 128)
+                                      for _ in range(2)])).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(H)
+    x = torch.empty((T, H), dtype=torch.bfloat16, device=DEV).normal_(generator=gen)
+    sel = torch.randint(0, 3, (T, 1), generator=gen, device=DEV)
+    rw = torch.rand((T, 1), generator=gen, device=DEV)
+    slots = {0: 1, 1: 0}
+    got = kernels.moe_prefill(pool, slots, x, sel, rw, n, H, I, bits)
+    for t in (slice(0, T // 2), slice(T // 2, T)):
+        want = kernels.moe_prefill(pool, slots, x[t], sel[t], rw[t], n, H, I, bits)
+        assert torch.equal(got[t].view(torch.int16), want.view(torch.int16))
+    # and against the bf16 weights in float32 on some tokens: products of bf16 values, one rounding of the activation and
+    # one of the result
+    some = torch.randint(0, T, (64,), generator=gen, device=DEV)
+    W = quant.dequant_rows(pool, torch.tensor([1, 0], device=DEV), n, bits, 128).float()
+    ref = torch.zeros((64, H), device=DEV)
+    for e in range(2):
+        g, u, d = W[e, 0].view(I, H), W[e, 1].view(I, H), W[e, 2].view(H, I)
+        xs = x[some].float()
+        a = (torch.nn.functional.silu(xs @ g.t()) * (xs @ u.t())).to(torch.bfloat16).float()
+        ref += (sel[some] == e) * rw[some] * (a @ d.t())
+    assert ((got[some].float() - ref).norm() / ref.norm()).item() <= 2.0**-7

@@ -1090,31 +1090,33 @@ __global__ __launch_bounds__(64 * kPlanWaves) void k_pf_plan(const ST* __restric
 // share a larger group's passes
 template <int BITS, int MT>
 static void launch_pf_mt(const Prefill& F, int ngroups, int max_group, hipStream_t st) {
-    // The LDS-DMA form takes an even number of K groups (a step is two, and a scale pair one aligned word) and x and
-    // act addressable with 32-bit offsets: every gate_up (H is a multiple of 256) and the down of an even I / 128.
+    // The LDS-DMA form takes an even number of K groups (a step is two, and a scale pair one aligned word) and an A operand
+    // of less than 2 GiB (32-bit offsets): every gate_up (H is a multiple of 256) whose x is, and the down of an even
+    // I / 128 whose act is.
     // 4-wave workgroups of 128 rows, token tiles staged per quant group: two or three workgroups share a CU (measured
     // on C5 against 8-wave workgroups with the tile staged per group pair, one per CU: T = 256 119.7 -> 114.3 us, 512
     // 150.5 -> 142.3). Against the register form, one call
     // with its plan and combine: 1,000 tokens over 64 experts of 4096 x 1536 at 4 bits (more than 16 K groups) 468 -> 274 us;
     // 2,000 tokens over 128 of 2048 x 768 449 -> 267 at 3 bits, 512 136 -> 104 at 2, 64 107 -> 92 at 3.
     const unsigned z = (unsigned)std::min(64, std::max(1, (max_group + MT * 16 - 1) / (MT * 16)));
-    const bool off32 = (int64_t)F.T * F.H * 2 < (int64_t(1) << 31) && (int64_t)F.P * F.I * 2 < (int64_t(1) << 31);
+    const bool x32 = (int64_t)F.T * F.H * 2 < (int64_t(1) << 31), act32 = (int64_t)F.P * F.I * 2 < (int64_t(1) << 31);
     Prefill G = F;
     G.gy = ngroups;
     G.gz = (int)z;
-    // the register form: passes of at most 4 tiles, 256 rows per workgroup
+    // the register form: passes of at most 4 tiles, 256 rows per workgroup (gate_up always of 4: from 16,384 tokens on)
     constexpr int MTR = MT > 4 ? 4 : MT;
     constexpr int NW = MTR >= 4 ? 8 : 4, RWG = 256;
+    const unsigned z4 = (unsigned)std::min(64, std::max(1, (max_group + 63) / 64));
     const unsigned zr = (unsigned)std::min(64, std::max(1, (max_group + MTR * 16 - 1) / (MTR * 16)));
-    const dim3 ggu((unsigned)(F.I / (RWG / 2)), (unsigned)ngroups, zr), gdn((unsigned)(F.H / RWG), (unsigned)ngroups, zr);
-    if (off32)
+    const dim3 ggu((unsigned)(F.I / (RWG / 2)), (unsigned)ngroups, z4), gdn((unsigned)(F.H / RWG), (unsigned)ngroups, zr);
+    if (x32)
         hipLaunchKernelGGL((k_pf_gate_up_dmag<BITS, MT, 4>), dim3((unsigned)(F.I / 64) * (unsigned)ngroups * z),
                            dim3(256), 0, st, G);
     else if (F.H / 128 <= kPfSmSteps)
-        hipLaunchKernelGGL((k_pf_gate_up<BITS, MTR, NW, RWG, true>), ggu, dim3(64 * NW), 0, st, F);
+        hipLaunchKernelGGL((k_pf_gate_up<BITS, 4, 8, RWG, true>), ggu, dim3(512), 0, st, F);
     else
-        hipLaunchKernelGGL((k_pf_gate_up<BITS, MTR, NW, RWG, false>), ggu, dim3(64 * NW), 0, st, F);
-    if (off32 && F.I / 128 % 2 == 0)
+        hipLaunchKernelGGL((k_pf_gate_up<BITS, 4, 8, RWG, false>), ggu, dim3(512), 0, st, F);
+    if (act32 && F.I / 128 % 2 == 0)
         hipLaunchKernelGGL((k_pf_down_dmag<BITS, MT, 4>), dim3((unsigned)(F.H / 128) * (unsigned)ngroups * z),
                            dim3(256), 0, st, G);
     else if (F.I / 128 <= kPfSmSteps)

@@ -442,29 +442,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // LDS-DMA form (an even number nk of K groups):
 // pf_gemm_dmag, k_pf_gate_up_dmag, k_pf_down_dmag.
 // A workgroup of 4 waves owns 128 weight rows, a wave 32 (two 16-row tiles).
-// A K step is one pair of groups (256 K): for each row the step's codes are one
-// whole 128-byte line at 4 bits (96 and 64 bytes at 3 and 2), and every line is fetched by ONE request:
-// global_load_lds_dwordx4 moves 64 lanes x 16 bytes = 8 rows x 128 bytes
-// straight into LDS (no VGPRs held while in flight), where each lane then reads
-// its MFMA fragment chunk. (Loads into registers in the fragment layout can only
-// cover 16 rows x 64 bytes per instruction, i.e. every line in two halves, which
-// measured 23 % slower in a loads-only run.)
-//   * codes: per wave one private slot (4 KB at 4 bits) + 256 B of the rows' fp16
+// A K step is one pair of groups (256 K). global_load_lds_dwordx4 moves 64 lanes x
+// 16 bytes straight into LDS (no VGPRs held while in flight), where each lane then
+// reads its MFMA fragment chunk. At 4 bits a row's step is one whole 128-byte line, and
+// an instruction covers 8 rows: every line is fetched by one request. (Loads into
+// registers in the fragment layout can only cover 16 rows x 64 bytes per instruction,
+// i.e. every line in two halves, which measured 23 % slower in a loads-only run.) At 2
+// bits a step is half a line of each of 16 rows, and the next step's request finds the
+// other half in L2 or not; at 3 bits it is 96 bytes, so that two steps share every other
+// line, and the requests follow the wave's 192 pieces in order, across rows.
+//   * codes: per wave one private slot (4, 3 or 2 KB) + 256 B of the rows' fp16
 //     scale and min pairs; it is read into registers at the step's start and
 //     then refilled with the next step's codes, which have the whole step to
 //     arrive.
 //   * tokens (A): the NT*16 rows x 256 bytes of one quant group, double-
 //     buffered, loaded by all waves (DMA as well) and published by a barrier
-//     per group. A workgroup holds 2 x NT*16*256 B + 17 KB of LDS, so three
-//     (NT = 4) or four (NT = 2) workgroups share a CU: measured on C5 at T = 512,
+//     per group. A workgroup holds 2 x NT*16*256 B and the four slots (17, 13 or 9 KB)
+//     of LDS, so three (NT = 4) or four (NT = 2) workgroups share a CU: measured on C5 at T = 512, 4 bits,
 //     three workgroups with one slot per wave beat two with two slots (125-129 µs
 //     against 142-145), the SIMDs' dequantisation, MFMA and LDS work then
 //     covering each other's waits.
 //   * A(2st+1) is issued before the step's code DMAs, so the step's one inner
 //     wait (for A(2st+1)) leaves the next step's codes in flight.
-//   * in LDS, piece p (16 bytes) of row r is stored at position p ^ (r & 7):
-//     the 8 lanes of a 128-bit LDS read phase (rows n..n+7, one piece) then hit
-//     8 different bank groups.
+//   * in LDS, piece p (16 bytes) of row r is stored at position p ^ (r & 7) (tokens, and
+//     codes at 4 bits; pf_code_offsets has the other widths'): the 8 lanes of a 128-bit
+//     LDS read phase (rows n..n+7, one piece) then hit 8 different bank groups.
 // The compiler neither emits nor counts these loads, so every wait for them is
 // an explicit s_waitcnt vmcnt(n), n = the number of DMA instructions this wave
 // issued after the awaited ones (vector memory loads complete in order), and

@@ -1154,8 +1154,12 @@ static void launch_gu(const Layer& L, const void* x, float* act, hipStream_t st)
 
 template <int BITS, int XT>
 static int gate_up_bits(const Layer& L, const void* x, float* act, hipStream_t st) {
-    // more than 64 chunks per row. Four chunks of a float32 x per lane take 170 registers: the generic kernel's one row per wave is as fast there
-    if (L.spr_gu > 64 && L.spr_gu <= (XT == WISP_DT_F32 ? 192 : 256) && L.gsh >= 2) {
+    // more than 64 chunks per row. Four chunks of a float32 x per lane take 170 registers: the generic kernel's one row per
+    // wave is as fast there. It is faster with a float32 x and few rows, whose lanes wait for their x longer: 4.45 us here
+    // against 3.60 at H 4096, k * I = 256, 4.48 against 4.08 at 512, 4.50 against 4.72 at 1,024 (2 bits 4.92 and 4.81) and
+    // 4.61 against 5.59 at 1,536; a bf16 x 3.24 against 3.90 at 256.
+    const bool few = XT == WISP_DT_F32 && (int64_t)L.k * L.I < (BITS == 2 ? 1025 : 1024);
+    if (L.spr_gu > 64 && L.spr_gu <= (XT == WISP_DT_F32 ? 192 : 256) && L.gsh >= 2 && !few) {
 #define WISP_GW(C, T)                                                                                               \
     hipLaunchKernelGGL((k_gate_up_wide<BITS, C, T, XT>), dim3((L.I + 4 * T - 1) / (4 * T), L.k), dim3(256), 0, st,  \
                        L.meta, L.pool, L.slot_bytes, L.nslots, x, act, L)

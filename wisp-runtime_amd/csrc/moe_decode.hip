@@ -1228,11 +1228,21 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
     const bool waves = L.k <= 16 && L.spr_dn <= 64 && L.gsh >= 0 &&
                        dn_lds_bytes(L, tuned ? tuning().dn_iters : 4) <= 65536;  // one wave per expert: k_down
     const int64_t pairs = (int64_t)L.k * L.spr_dn;
-    // k_down_wide keeps every lane at work and needs no particular k; k_down stages a quarter of the activations per
-    // row and stays where it can run (`waves`) with few output rows and many pairs: layers of 2,048 rows at k = 8 took
-    // 10.05 us with it against 10.35 (I 1024) and 11.6 against 12.0 (I 1408, k = 6), and 8.6 against 8.5 (I 1024, k = 5),
-    // 13.1 against 11.3 (3,072 rows, I 1152, k = 4) the other way. I = 768 keeps its tuned forms.
-    if (WSUM && L.gsh >= 2 && pairs <= 512 && !(waves && (tuned || (L.H <= 2048 && pairs > 192)))) {
+    // k_down_wide needs no particular k, keeps every lane at work and gives a row one wave of its own, NC steps of 64 pairs
+    // with the sums over LDS; k_down, where it can run (`waves`), is a wave per expert and 4 (64 / (I/32)) rows, k / (64 /
+    // (I/32)) steps a row. The bits are the same, so the steps and the rows decide: with few rows both are one round of
+    // waves and the shorter chain is k_down_wide's, up to three or four steps; with many rows the steps count, where k_down's
+    // are cheaper (its activations stay in registers for four rows), less so at 2 bits. Fitted over 2,268 shapes (H 512 to
+    // 8,192, I 128 to 2,048, k 1 to 16, three widths): within 1 % of the better kernel on average, k_down alone 11 % off,
+    // k_down_wide alone 4 %. us a call, 4 bits, wide / k_down: H 512, I 384, k 8 3.3 / 4.4; H 4096, I 256, k 6 3.8 / 4.3; H 3072, I 1152, k 5 5.6 / 5.8,
+    // k 8 8.5 / 7.6; H 2048, I 1024, k 8 5.5 / 4.7; H 5120, I 1408, k 6 12.4 / 10.9; H 4096, I 1536, k 8 10.5 / 10.5 (2 bits
+    // 9.3 / 10.9). I = 768 keeps its tuned forms.
+    const int NC = pairs <= 256 ? (int)(pairs + 63) / 64 : pairs <= 384 ? 6 : pairs <= 448 ? 7 : 8;
+    const float steps_dn = waves ? (float)L.k / (float)(64 / L.spr_dn) : 0.f;
+    const float more = NC - (BITS == 2 ? 0.7f : 0.6f) * steps_dn;  // k_down_wide's steps beyond k_down's, in its own
+    const bool wide = (more * L.H <= (BITS == 2 ? 3500.f : 3000.f) || (more <= 0.5f && L.k > 2)) &&
+                      !(L.H <= 2048 && NC > (L.H <= 1024 ? 4 : 3));
+    if (WSUM && L.gsh >= 2 && pairs <= 512 && (!waves || (wide && !tuned))) {
         const int lsh = waves ? __builtin_ctz(lanes_per_sum(4 * (64 / L.spr_dn))) : 4;  // k_down sums 4 row iterations
         const bool n8 = L.H >= 4096;  // eight rows per staged activation once that still leaves two workgroups per CU
 #define WISP_DWO(C, NWV, WV)                                                                                   \

@@ -870,11 +870,10 @@ __global__ __launch_bounds__(1024) void k_down_c2(const float* meta, const uint8
 // LDS, and each expert's are added, weighted and summed over the experts as the kernel that takes the shape otherwise does
 // it, so the bits are the same whatever the weights hold: WAVES in k_down's order (group_sum over 2^lsh_dn lanes, the products
 // rounded), else in k_down_generic's (the butterfly over 64 chunk columns, in rows of 16 lanes; fma). Bound by VALU
-// issue and, in the small shapes, by the chain of round trips. A layer (both kernels, 4 bits) of H 4096, I 1536, k = 8 takes
-// 22.9 us, 27.0 with the general kernels (k_down: a wave per expert, 48 of 64 lanes at work, the activations staged per 4
-// rows); H 5120, I 1408, k = 10 35.2 and 69.9; H 512, I 384, k = 8 6.7 and 7.7. Weighting each pair and summing the wave
-// once instead took 22.7, 34.5 and 6.0, in another order, and gave NaN for an infinite weight (0 times it in lanes without a
-// pair). Two rows per wave spill at NC = 8.
+// issue and, in the small shapes, by the chain of round trips. A layer (both kernels, 4 bits) of H 5120, I 1408, k = 10
+// takes 33.7 us, 69.9 with the general kernels; H 512, I 384, k = 8 6.2 and 7.4; H 4096, I 256, k = 6 7.6 and 9.95. Weighting
+// each pair and summing the wave once instead took 33.3, 5.8 and 7.3, in another order, and gave NaN for an infinite weight
+// (0 times it in lanes without a pair). Two rows per wave spill at NC = 8.
 template <int BITS, int NC, int NWV, bool WAVES>
 __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const uint8_t* __restrict__ pool,
                                                         int64_t slot_bytes, int nslots, int k,
@@ -956,81 +955,66 @@ __global__ __launch_bounds__(64 * NWV) void k_down_wide(const float* meta, const
 #pragma unroll
     for (int c = 0; c < NC; ++c) part[min(lane + 64 * c, total - 1)] = p[c];
     wave_sync_lds();
-    // 2^lsh lanes sum an expert; two rounds of EPR experts at a time, their reads in flight together. What lies past a row
-    // or past the last expert adds +0 to sums that started at +0: no change, whatever they hold.
+    // 2^lsh lanes sum an expert, EPR experts a round. What lies past a row or past the last expert adds +0 to sums that
+    // started at +0: no change, whatever they hold. The first two rounds' reads are in flight together.
     float acc = 0.f;
-    for (int e0 = 0; e0 < k; e0 += 2 * EPR) {
-        const bool two = e0 + EPR < k;
-        int e[2];
-        const float* pe[2];
-        float v[2];
+    // the sum of expert e's values: t holds the lane's, requested by get
+    constexpr int M = WAVES ? 6 : 4;  // WAVES: all of a row's (I / 32 <= 64, in lanes_per_sum's lanes); else 64 columns' worth
+    auto get = [&](int e, int i0, float* t) {
+        const float* pe = part + min(e, k - 1) * SPR;
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            e[r] = e0 + r * EPR + (lane >> lsh);
-            pe[r] = part + min(e[r], k - 1) * SPR;
-            if (e0) wr[r] = meta[k + min(e[r], k - 1)];
-        }
+        for (int u = 0; u < M; ++u) t[u] = pe[min(i0 + (u << lsh) + sub, SPR - 1)];
+    };
+    auto sum = [&](int e, float* t) {
+        float v = 0.f;
         if constexpr (WAVES) {  // group_sum's strided form
-            v[0] = v[1] = 0.f;
-            for (int i0 = sub; i0 - sub < SPR; i0 += 4 << lsh) {
-                float t[2][4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) t[0][u] = pe[0][min(i0 + (u << lsh), SPR - 1)];
-                if (two)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) t[1][u] = pe[1][min(i0 + (u << lsh), SPR - 1)];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[0] += i0 + (u << lsh) < SPR ? t[0][u] : 0.f;
-                if (two)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) v[1] += i0 + (u << lsh) < SPR ? t[1][u] : 0.f;
-            }
-            if (lsh >= 1) { v[0] += dpp_f<0xB1>(v[0]); v[1] += dpp_f<0xB1>(v[1]); }
-            if (lsh >= 2) { v[0] += dpp_f<0x4E>(v[0]); v[1] += dpp_f<0x4E>(v[1]); }
-            if (lsh >= 3) { v[0] += dpp_f<0x141>(v[0]); v[1] += dpp_f<0x141>(v[1]); }
-            if (lsh >= 4) { v[0] += dpp_f<0x140>(v[0]); v[1] += dpp_f<0x140>(v[1]); }
+            for (int u = 0; u < M; ++u) v += (u << lsh) + sub < SPR ? t[u] : 0.f;
+            v += lsh >= 1 ? dpp_f<0xB1>(v) : 0.f;
+            v += lsh >= 2 ? dpp_f<0x4E>(v) : 0.f;
+            v += lsh >= 3 ? dpp_f<0x141>(v) : 0.f;
+            v += lsh >= 4 ? dpp_f<0x140>(v) : 0.f;
         } else {  // wave_sum over 64 columns: steps 32 and 16 between a lane's four, then 8, 4, 2, 1 within the row
-            float s[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-            for (int i0 = sub; i0 - sub < SPR; i0 += 64) {
-                float t[2][4];
+            float s[4];
 #pragma unroll
-                for (int r = 0; r < 2; ++r)
+            for (int q = 0; q < 4; ++q) s[q] = 0.f + (16 * q + sub < SPR ? t[q] : 0.f);
+            for (int i0 = 64; i0 < SPR; i0 += 64) {
+                get(e, i0, t);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) t[r][q] = pe[r][min(i0 + 16 * q, SPR - 1)];
-#pragma unroll
-                for (int r = 0; r < 2; ++r)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) s[r][q] += i0 + 16 * q < SPR ? t[r][q] : 0.f;
+                for (int q = 0; q < 4; ++q) s[q] += i0 + 16 * q + sub < SPR ? t[q] : 0.f;
             }
-#pragma unroll
-            for (int r = 0; r < 2; ++r) v[r] = (s[r][0] + s[r][2]) + (s[r][1] + s[r][3]);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                v[r] += dpp_f<0x128>(v[r]);
-                v[r] += dpp_f<0x124>(v[r]);
-                v[r] += dpp_f<0x122>(v[r]);
-                v[r] += dpp_f<0x121>(v[r]);
-            }
+            v = (s[0] + s[2]) + (s[1] + s[3]);
+            v += dpp_f<0x128>(v);
+            v += dpp_f<0x124>(v);
+            v += dpp_f<0x122>(v);
+            v += dpp_f<0x121>(v);
         }
+        return e < k ? v : 0.f;
+    };
+    auto add = [&](int e0, float v, float w) {  // experts e0 .. e0 + EPR - 1, in order
+        if constexpr (WAVES) v = w * v;
+        for (int g = 0; g < EPR && e0 + g < k; g += 4)
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            wr[r] = e[r] < k ? wr[r] : 0.f;
-            v[r] = e[r] < k ? v[r] : 0.f;
-            if constexpr (WAVES) v[r] = wr[r] * v[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-            for (int g = 0; g < EPR && e0 + r * EPR + g < k; g += 4)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const float ve = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[r]), (g + u) << lsh));
-                    if constexpr (WAVES) {
-                        acc = add_rn(acc, ve);
-                    } else {
-                        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wr[r]), (g + u) << lsh));
-                        acc = __builtin_fmaf(w, ve, acc);
-                    }
+            for (int u = 0; u < 4; ++u) {
+                const float ve = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (g + u) << lsh));
+                if constexpr (WAVES) {
+                    acc = add_rn(acc, ve);
+                } else {
+                    const float we = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), (g + u) << lsh));
+                    acc = __builtin_fmaf(we, ve, acc);
                 }
+            }
+    };
+    const int el = lane >> lsh;
+    float t0[M], t1[M];
+    get(el, 0, t0);
+    if (EPR < k) get(EPR + el, 0, t1);
+    add(0, sum(el, t0), el < k ? wr[0] : 0.f);
+    if (EPR < k) add(EPR, sum(EPR + el, t1), EPR + el < k ? wr[1] : 0.f);
+    for (int e0 = 2 * EPR; e0 < k; e0 += EPR) {
+        const float w = meta[k + min(e0 + el, k - 1)];
+        get(e0 + el, 0, t0);
+        add(e0, sum(e0 + el, t0), e0 + el < k ? w : 0.f);
     }
     if (lane == 0 && h < L.H) store_out(out, L.odt, h, acc);
 }
@@ -1233,10 +1217,11 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
     // (I/32)) steps a row. The bits are the same, so the steps and the rows decide: with few rows both are one round of
     // waves and the shorter chain is k_down_wide's, up to three or four steps; with many rows the steps count, where k_down's
     // are cheaper (its activations stay in registers for four rows), less so at 2 bits. Fitted over 2,268 shapes (H 512 to
-    // 8,192, I 128 to 2,048, k 1 to 16, three widths): within 1 % of the better kernel on average, k_down alone 11 % off,
-    // k_down_wide alone 4 %. us a call, 4 bits, wide / k_down: H 512, I 384, k 8 3.3 / 4.4; H 4096, I 256, k 6 3.8 / 4.3; H 3072, I 1152, k 5 5.6 / 5.8,
-    // k 8 8.5 / 7.6; H 2048, I 1024, k 8 5.5 / 4.7; H 5120, I 1408, k 6 12.4 / 10.9; H 4096, I 1536, k 8 10.5 / 10.5 (2 bits
-    // 9.3 / 10.9). I = 768 keeps its tuned forms.
+    // 8,192, I 128 to 2,048, k 1 to 16, three widths): within 1 % of the better kernel on average, k_down alone 14 % off,
+    // k_down_wide alone 3 %. us a call, 4 bits, wide / k_down: H 512, I 384, k 8 3.1 / 4.4; H 4096, I 256, k 6
+    // 3.5 / 4.3; H 3072, I 1152, k 5 5.7 / 5.9, k 8 8.6 / 7.6; H 2048, I 1024, k 8 5.3 / 4.7; H 5120, I 1408,
+    // k 6 12.4 / 11.0; H 8192, I 256, k 1 4.5 / 3.4; H 4096, I 1536, k 8 10.4 / 10.4 (2 bits 9.3 / 10.8). I = 768
+    // keeps its tuned forms.
     const int NC = pairs <= 256 ? (int)(pairs + 63) / 64 : pairs <= 384 ? 6 : pairs <= 448 ? 7 : 8;
     const float steps_dn = waves ? (float)L.k / (float)(64 / L.spr_dn) : 0.f;
     const float more = NC - (BITS == 2 ? 0.7f : 0.6f) * steps_dn;  // k_down_wide's steps beyond k_down's, in its own

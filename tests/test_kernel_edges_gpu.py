@@ -130,7 +130,10 @@ def _group_64(rows, n, bits):
 @pytest.mark.parametrize("bits", [4, 3, 2])
 @pytest.mark.parametrize("H,I,k", [(4096, 1536, 8), (2176, 128, 1), (4224, 256, 17), (6272, 128, 2), (8192, 128, 2),
                                    (384, 1152, 5), (384, 1024, 3), (384, 640, 9), (384, 512, 16), (640, 384, 16),
-                                   (384, 128, 65), (384, 8192, 2), (384, 2304, 7), (5120, 1408, 10)])
+                                   (384, 128, 65), (384, 8192, 2), (384, 2304, 7), (5120, 1408, 10), (4096, 1536, 4),
+                                   (4096, 1280, 6), (4096, 1152, 10), (3072, 1152, 10), (4096, 1536, 10), (384, 1536, 4),
+                                   (2176, 896, 2), (4096, 256, 8), (4096, 640, 3), (3072, 1792, 7), (4096, 384, 40), (384, 128, 17),
+                                   (384, 128, 40), (384, 128, 60), (4096, 128, 60), (4096, 128, 90)])
 def test_wide_decode_layers_equal_the_general_kernels(bits, H, I, k):
     rng = np.random.default_rng(H + I + k + bits)
     n, E = H * I, k + 1

@@ -1226,7 +1226,7 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
     const float steps_dn = waves ? (float)L.k / (float)(64 / L.spr_dn) : 0.f;
     const float more = NC - (BITS == 2 ? 0.7f : 0.6f) * steps_dn;  // k_down_wide's steps beyond k_down's, in its own
     const bool wide = (more * L.H <= (BITS == 2 ? 3500.f : 3000.f) || (more <= 0.5f && L.k > 2)) &&
-                      !(L.H <= 2048 && NC > (L.H <= 1024 ? 4 : 3));
+                      !(L.H <= 2048 && NC > (L.H <= 1024 ? 4 : 3)) && NC <= 6;
     if (WSUM && L.gsh >= 2 && pairs <= 512 && (!waves || (wide && !tuned))) {
         const int lsh = waves ? __builtin_ctz(lanes_per_sum(4 * (64 / L.spr_dn))) : 4;  // k_down sums 4 row iterations
         const bool n8 = L.H >= 4096;  // eight rows per staged activation once that still leaves two workgroups per CU
@@ -1239,7 +1239,7 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
         if (waves) WISP_DWO(C, NWV, true); \
         else WISP_DWO(C, NWV, false);   \
     } while (0)
-        if (pairs <= 64) WISP_DW(1, 4);
+        if (pairs <= 64) WISP_DWO(1, 4, true);  // so few are always k_down's to take too
         else if (pairs <= 128) WISP_DW(2, 4);
         else if (pairs <= 192 && n8) WISP_DW(3, 8);
         else if (pairs <= 192) WISP_DW(3, 4);
@@ -1247,9 +1247,9 @@ static int down_bits(const Layer& L, const float* act, void* out, float* y, hipS
         else if (pairs <= 256) WISP_DW(4, 4);
         else if (pairs <= 384 && n8) WISP_DW(6, 8);
         else if (pairs <= 384) WISP_DW(6, 4);
-        else if (pairs <= 448 && n8) WISP_DW(7, 8);
-        else if (n8) WISP_DW(8, 8);
-        else WISP_DW(8, 4);
+        else if (pairs <= 448 && n8) WISP_DWO(7, 8, false);  // k_down stays where it can run with so many
+        else if (n8) WISP_DWO(8, 8, false);
+        else WISP_DWO(8, 4, false);
 #undef WISP_DW
 #undef WISP_DWO
         return check_launch("k_down_wide");

@@ -772,7 +772,7 @@ def summarize_c5(runs, cmds) -> str:
         ex = [p["experts_touched"] for p in res["config"]["per_T"] if p["T"] == T][0]
         with open(stats_csv) as f:
             rows = [r for r in csv.DictReader(f) if "k_pf" in r["Name"]]
-        for r in sorted(rows, key=lambda r: ("gate_up" not in r["Name"], "combine" in r["Name"])):
+        for r in sorted(rows, key=lambda r: ("plan" not in r["Name"], "gate_up" not in r["Name"], "combine" in r["Name"])):
             name = r["Name"].split("(")[0].replace("void ", "")
             wb = ex * (gu_w if "gate_up" in name else dn_w if "down" in name else 0)
             avg = float(r["AverageNs"])
@@ -893,10 +893,12 @@ def run_c4(a) -> dict:
 # ----------------------------------------------------------------------------- C5: grouped prefill
 def run_c5(a) -> dict:
     """Config 5: chunked-prefill grouped dequant-GEMM. T tokens, each routed top-8 over 128
-    experts by Zipf(1.1); per-expert token groups run the 4-bit dequant-into-LDS + bf16 MFMA
-    kernels (gate_up+SiLU, down, combine). Experts are resident in slot pools rotated past
-    the Infinity Cache; the three launches per chunk are captured in a graph and timed with
-    HIP events."""
+    experts by Zipf(1.1), through kernels.moe_prefill with the routing on the GPU: the plan and
+    the 4-bit dequant-into-LDS + bf16 MFMA kernels (gate_up+SiLU, down, combine). Experts are
+    resident in slot pools rotated past the Infinity Cache; the four launches per chunk are
+    captured in a graph and timed with HIP events. --c5-plan host: the three launches of the
+    C entry on work items planned on the host beforehand, as a call with the routing in host
+    memory runs them."""
     import numpy as np
 
     from wisp import kernels as K
@@ -927,7 +929,13 @@ def run_c5(a) -> dict:
         out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
         ng = len(uniq)
 
+        seld, wd = torch.from_numpy(sel).to(dev), w.to(dev)
+        slots = [{e: e + l * E for e in range(E)} for l in range(P_)]
+
         def launch(l, st):
+            if a.c5_plan == "gpu":
+                K.moe_prefill(W.pool, slots[l], x, seld, wd, H * I, H, I, a.bits, G)
+                return
             ints = plans[l]
             _lib.check(L.wisp_moe_prefill(
                 _lib.ptr(W.pool), nb, W.pool.shape[0], _lib.ptr(ints), ng, int(count.max()), _lib.ptr(ints[ng * 3:]),
@@ -955,7 +963,7 @@ def run_c5(a) -> dict:
         t = statistics.median(replay_seconds(W.stream, g, reps) for _ in range(5)) / (reps * P_)
         flops = T * K_TOP * 6 * H * I
         byts = ng_experts * nb + 2 * T * H + 2 * 2 * Pn * I + 2 * 4 * Pn * H + 2 * T * H
-        out_rows.append({"T": T, "experts_touched": ng_experts, "work_items": ng, "us": round(t * 1e6, 2),
+        out_rows.append({"T": T, "experts_touched": ng_experts, "work_items": ng if a.c5_plan == "host" else None, "us": round(t * 1e6, 2),
                          "TFLOP/s": round(flops / t / 1e12, 2), "mfma_util": round(flops / t / 1e12 / peak_tflops, 4),
                          "GB/s": round(byts / t / 1e9, 1), "hbm_frac": round(byts / t / 1e9 / PEAK_HBM_GBS, 4),
                          "bytes": byts, "flops": flops})
@@ -975,6 +983,7 @@ def run_c5(a) -> dict:
         "dtype": "bf16",
         "data": "synthetic",
         "config": {"workload": f"C5: T in {a.c5_tokens}, H={H} I={I}, {a.c5_pools} expert pools rotated",
+                   "plan": a.c5_plan,
                    "timing": "per T: one graph of the pools' launches; `warmup` untimed replays, then the "
                              "median of 5 HIP-event timings of `steps` replays",
                    "per_T": out_rows},
@@ -1235,7 +1244,10 @@ def main():
     ap.add_argument("--gptoss-reps", type=int, default=50, help="timed replays of the rotated layers")
     ap.add_argument("--c5-pools", type=int, default=8)
     ap.add_argument("--c5-reps", type=int, default=10)
-    ap.add_argument("--c5-chunk", type=int, default=0, help="pairs per prefill work item (0: the package default)")
+    ap.add_argument("--c5-plan", default="gpu", choices=["gpu", "host"],
+                    help="gpu: kernels.moe_prefill, the pairs grouped on the GPU; host: work items planned beforehand")
+    ap.add_argument("--c5-chunk", type=int, default=0,
+                    help="pairs per prefill work item of --c5-plan host (0: the package default)")
     ap.add_argument("--c4-layers", type=int, default=48)
     ap.add_argument("--c4-slots", type=int, default=512)
     ap.add_argument("--c4-tokens", type=int, default=32)

@@ -92,8 +92,9 @@ def test_attn_decode_short_context_in_a_large_cache(Hq, Hk, D):
     assert ((got - ref).norm() / ref.norm()).item() <= 2.0**-8  # one bf16 rounding and fp32 sums
 
 
-# kernel 1 rows of 2, 3 and 4 chunks per lane (a remainder in each; float32 x of four goes to the generic kernel),
-# kernel 2 with 4 to 512 (expert, chunk) pairs: part of one step, every step count, and more than 16 experts
+# kernel 1 rows of 2, 3 and 4 chunks per lane (a remainder in each; float32 x of four, or of few rows, goes to the generic
+# kernel), kernel 2 with 4 to 512 (expert, chunk) pairs and more than 16 experts, whichever kernel the rules give them
+# (the next test has every form of the wide ones)
 @pytest.mark.parametrize("bits", [4, 3, 2])
 @pytest.mark.parametrize("H,I,group,k", [(2176, 128, 128, 1), (4096, 256, 256, 3), (4224, 128, 128, 17), (6272, 128, 128, 2),
                                          (8192, 128, 128, 2), (256, 640, 128, 5), (4096, 512, 256, 13), (256, 1152, 128, 6),

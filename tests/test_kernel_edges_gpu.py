@@ -145,7 +145,7 @@ def test_wide_decode_layers_equal_the_general_kernels(bits, H, I, k):
     for last in (w[-1], np.float32("inf"), np.float32("-inf"), np.float32("nan")):
         w[-1] = last
         meta = torch.from_numpy(O.meta(slots, w)).to(DEV)
-        for xdt in (torch.bfloat16, torch.float32):
+        for xdt in (torch.bfloat16, torch.float16, torch.float32):
             x = torch.from_numpy(rng.standard_normal(H).astype(np.float32)).to(xdt).to(DEV)
             got = kernels.moe_decode_fast(p128, meta, x, k, n, H, I, bits, 128)
             want = kernels.moe_decode_fast(p64, meta, x, k, n, H, I, bits, 64)
